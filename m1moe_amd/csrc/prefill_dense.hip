@@ -18,10 +18,11 @@
 //   rope_kv_rows   per token and head: the per-head q/k RMSNorm and RoPE at
 //                  the token's position (InferenceEngine.swift:521-548), k and
 //                  v rows into the caches (:215-220)
-//   attn_mfma      causal attention of the T queries over positions 0 .. their
-//                  own (Shaders.metal:209-326 for every token) on f32 MFMA,
-//                  online softmax over key blocks staged in LDS (head_dim 64,
-//                  128; attn_causal, on the SIMD units, for head_dim 256)
+//   attn_split     causal attention of the T queries over positions 0 .. their
+//                  own (Shaders.metal:209-326 for every token) on bf16 MFMA
+//                  with the f32 operands split exactly, online softmax over
+//                  key blocks (head_dim 64, 128; attn_causal, on the SIMD
+//                  units, for head_dim 256)
 //
 // The MoE block runs through the grouped prefill (prefill.hip).
 #include <hip/hip_runtime.h>
@@ -541,152 +542,330 @@ int launch_pf_rope_kv(const PfDenseArgs& a, void* stream) {
     return (int)hipGetLastError();
 }
 
-// Causal attention on v_mfma_f32_16x16x4f32 (f32 operands and accumulation;
-// head_dim 64 or 128).  Workgroup = (head, 64 queries), wave = 16 queries.
-// Keys go in blocks of 32 through LDS, shared by the four waves: K row-major,
-// V transposed.  Per block a wave computes S = Q K^T (16 x 32), updates each
-// query row's running max and sum (the softmax of Shaders.metal:245-289 in
-// pieces), writes P = e^(S - m) to LDS and reads it back as the A operand of
-// O += P V.  Contraction orders: in k-step 4t+u lane (r, kq) supplies dim (or
-// key) 16t + 4kq + u, so each lane's four steps read 16 contiguous bytes.
+// ---- causal attention on bf16 MFMA with f32 operands split three ways ----------------
+
+// Three bf16 parts of eight f32 values, two per word: hi = bf16(x), mid =
+// bf16(x - hi), lo = bf16(x - hi - mid), each rounded to nearest: 24
+// significant bits, so the parts add up to x exactly.  The differences of a
+// pair are one v_dot2 each, (hi0, hi1) . (-1, 0) + x0 and (hi0, hi1) . (0, -1)
+// + x1 (exact: the result fits f32), 3.5 instructions per value against 5.5
+// with the parts unpacked and subtracted.  The constants live in scalar
+// registers: as literals the compiler makes them inline operands, which the
+// instruction reads as f32, not as a bf16 pair.
+struct Split8 {
+    bf16x8 h, m, l;
+};
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ Split8 split8_rne(const float (&v)[8]) {
+    uint32_t c0, c1;
+    asm("s_mov_b32 %0, 0xbf80" : "=s"(c0));
+    asm("s_mov_b32 %0, 0xbf800000" : "=s"(c1));
+    const bf16x2 n0 = __builtin_bit_cast(bf16x2, c0), n1 = __builtin_bit_cast(bf16x2, c1);
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x0 = v[2 * i], x1 = v[2 * i + 1];
+        const bf16x2 hi = __builtin_convertvector(f32x2v{x0, x1}, bf16x2);
+        const float r0 = __builtin_amdgcn_fdot2_f32_bf16(hi, n0, x0, false);
+        const float r1 = __builtin_amdgcn_fdot2_f32_bf16(hi, n1, x1, false);
+        const bf16x2 mid = __builtin_convertvector(f32x2v{r0, r1}, bf16x2);
+        const float t0 = __builtin_amdgcn_fdot2_f32_bf16(mid, n0, r0, false);
+        const float t1 = __builtin_amdgcn_fdot2_f32_bf16(mid, n1, r1, false);
+        h[i] = __builtin_bit_cast(uint32_t, hi);
+        m[i] = __builtin_bit_cast(uint32_t, mid);
+        l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2v{t0, t1}, bf16x2));
+    }
+    Split8 s;
+    s.h = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
+    s.m = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
+    s.l = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
+    return s;
+}
+
+// acc += A B over 16 contraction slots with both f32 operands split: the six
+// part products down to 2^-16 of the largest, small ones first.  The three
+// left out are below 2^-23 of a product (2^-25 on average, either sign):
+// less than the rounding of an f32 product.
+__device__ __forceinline__ void mfma_split(const Split8& a, const Split8& b, f32x16v& acc) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l, b.h, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.l, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.m, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.h, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.m, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.h, acc, 0, 0, 0);
+}
+
+__device__ __forceinline__ float halves_max(float v) {  // lanes l and l ^ 32
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float halves_add(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// One wave's 32 queries of one head: its running softmax and the transposed
+// output accumulators.  Lane l holds query l % 32 (both halves the same one):
+// of the scores S^T = K Q^T of a 32-key block the 16 keys 8 (v / 4) + 4 h + v
+// % 4 (h = l / 32), of O^T (NT tiles of 32 rows) the rows in the same order;
+// dim NT r + t of the head is row r of tile t, so that a lane's V and output
+// values of all tiles are NT consecutive floats.
+// Contraction slots: lane half h, element e of k-step s is dim (or key) 16 s
+// + 4 h + e for e < 4 and 16 s + 8 + 4 h + e - 4 above: the accumulator's row
+// order, so P multiplies V straight from the lanes that computed it.
 template <int HD>
-__global__ __launch_bounds__(256) void attn_mfma_kernel(PfDenseArgs a) {
-    constexpr int QW = 16, QB = 64, KB = 32;
-    constexpr int NT = HD / 16;  // 16-wide dim groups: Q K^T k-step groups, output blocks
-    __shared__ __attribute__((aligned(16))) float sK[KB][HD + 4];
-    __shared__ __attribute__((aligned(16))) float sVt[HD][KB + 4];
-    __shared__ __attribute__((aligned(16))) float sP[4][QW][KB + 4];
-    const int h = blockIdx.x, tb = blockIdx.y * QB;
+struct AttnWave {
+    static constexpr int NT = HD / 32, NS = HD / 16;
+    typedef float vecT __attribute__((ext_vector_type(NT)));
+    const float *qrow, *kbase, *vbase;   // the lane's query; the kv head's columns
+    int kvd, r32, h, t, qpos, first, last, nblk;
+    float c, m, l;                       // c = scale log2(e); m the running maximum of the raw scores
+    f32x16v acc[NT];
+
+    __device__ __forceinline__ void init(const PfDenseArgs& a, int head, int t0, int lane) {
+        const int p0 = *a.pos, kvh = head / a.hpkv;
+        r32 = lane & 31;
+        h = lane >> 5;
+        kvd = a.kvd;
+        c = a.scale * 1.44269504088896341f;
+        t = min(t0 + r32, a.T - 1);
+        qpos = min(p0 + t, a.max_seq - 1);
+        first = min(p0 + t0, a.max_seq - 1);                       // the tile's first and
+        last = min(p0 + min(t0 + 31, a.T - 1), a.max_seq - 1);     // last query position
+        nblk = last / 32 + 1;
+        qrow = a.qkv + (size_t)t * a.ldqkv + (size_t)head * HD;
+        kbase = a.kcache + (size_t)kvh * HD;
+        vbase = a.vcache + (size_t)kvh * HD;
+        clear();
+    }
+    __device__ __forceinline__ void clear() {
+        m = -INFINITY;
+        l = 0.f;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
+    }
+    // k-step s of the lane's query, split
+    __device__ __forceinline__ Split8 query(int s) const {
+        const float4 x0 = *reinterpret_cast<const float4*>(qrow + 16 * s + 4 * h);
+        const float4 x1 = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 + 4 * h);
+        return split8_rne({x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w});
+    }
+    // The running softmax (Shaders.metal:245-289 in pieces) over the lane's 16
+    // keys and the other half's: s becomes the numerators, acc is rescaled.  m
+    // is the largest raw score; e^((s - m) scale) = 2^(s c - m c), c = scale
+    // log2(e), one fused multiply-add (one rounding) and the hardware exp2.
+    __device__ __forceinline__ void softmax(int k0, f32x16v& s) {
+        if (k0 + 31 > first) {   // (uniform) some query of the tile does not see the whole block
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                s[v] = k0 + 8 * (v >> 2) + 4 * h + (v & 3) <= qpos ? s[v] : -INFINITY;
+        }
+        float bm = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) bm = fmaxf(bm, s[v]);
+        const float mn = fmaxf(m, halves_max(bm));
+        const float mc = mn == -INFINITY ? 0.f : mn * c;   // (no key seen yet: every numerator 0)
+        const float f = __builtin_amdgcn_exp2f(fmaf(m, c, -mc));
+        float ls = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            s[v] = __builtin_amdgcn_exp2f(fmaf(s[v], c, -mc));
+            ls += s[v];
+        }
+        l = fmaf(l, f, ls);
+        m = mn;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][v] *= f;
+    }
+    // Whether some score (odd: a sum of them times 0) or output of the wave is
+    // not finite: an infinity or NaN among its q, k and v, or a value so
+    // large that its bf16 part rounds to infinity (its parts then add up to NaN).
+    __device__ __forceinline__ bool not_finite(float odd) const {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) odd = fmaf(acc[i][v], 0.f, odd);
+        return __any(odd != 0.f);
+    }
+    // Blocks b0, b0 + step, ... again on f32 MFMA, for such a wave: lane half h
+    // supplies dims 8 j + 4 h + e of Q and K, then the lane's own keys of P.
+    __device__ __forceinline__ void f32_blocks(int b0, int step) {
+        clear();
+#pragma unroll 1
+        for (int b = b0; b < nblk; b += step) {
+            const int k0 = 32 * b;
+            f32x16v s;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll 1
+            for (int j = 0; j < 2 * NS; ++j) {
+                const float4 q = *reinterpret_cast<const float4*>(qrow + 8 * j + 4 * h);
+                const float4 k = *reinterpret_cast<const float4*>(
+                    kbase + (size_t)min(k0 + r32, last) * kvd + 8 * j + 4 * h);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.x, q.x, s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.y, q.y, s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.z, q.z, s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.w, q.w, s, 0, 0, 0);
+            }
+            softmax(k0, s);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const vecT x = *reinterpret_cast<const vecT*>(
+                    vbase + (size_t)min(k0 + 8 * (v >> 2) + 4 * h + (v & 3), last) * kvd + NT * r32);
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i], s[v], acc[i], 0, 0, 0);
+            }
+        }
+    }
+};
+
+// Causal attention, head_dim 64 or 128, on v_mfma_f32_32x32x16_bf16 with the
+// f32 operands split (mfma_split): six bf16 MFMAs in place of one f32 MFMA at
+// a sixteenth of the rate.  Workgroup = (head, 32 queries); wave w takes key
+// blocks w, w + 4, ... with a running softmax of its own, the four merged
+// through LDS at the end.  K and V come straight from the cache into the lanes
+// that split and multiply them: no barrier in the loop, and heads x T / 32
+// workgroups, so a short prompt still spreads over the chip.  Before, 64
+// queries per workgroup on f32 MFMA with K and V staged in LDS: 16 heads of
+// 128, T = 128 26.1 -> 10.5 us, T = 333 65.4 -> 17.4; 32 q / 8 kv heads, T =
+// 2048 632 -> 285 us.  Bound at long prompts by the vector unit (the splits of
+// K and V, ~800 instructions per 96 MFMAs) and the K loads' 32-byte pieces
+// (data return busy 78% of the time).  128 queries per workgroup sharing
+// each block's split through LDS took 255 us there (eight waves; their
+// barriers keep the splits and the MFMAs of a SIMD's two waves in step), the
+// same as this form at T = 1500 and 132 -> 178 us at 16 heads, T = 2000.
+template <int HD>
+__global__ __launch_bounds__(256, 2) void attn_split_kernel(PfDenseArgs a) {
+    constexpr int NT = HD / 32, NS = HD / 16;
+    typedef typename AttnWave<HD>::vecT vecT;
+    // the split queries (an operand image per part and k-step), then the
+    // waves' partial outputs
+    constexpr int kQBytes = 3 * NS * 64 * 16, kOBytes = 4 * 16 * NT * 64 * 4;
+    __shared__ __attribute__((aligned(16))) uint8_t s_buf[kQBytes > kOBytes ? kQBytes : kOBytes];
+    __shared__ float s_m[4][32], s_l[4][32];
+    bf16x8* sQ = reinterpret_cast<bf16x8*>(s_buf);  // [3][NS][64]
+    float* sO = reinterpret_cast<float*>(s_buf);    // [4][16 NT][64]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int lr = lane & 15, kq = lane >> 4;
-    const int p0 = *a.pos;
-    const int kvh = h / a.hpkv;
-    const int qw0 = tb + wave * QW;  // the wave's first query (token index)
-    // the workgroup's last query position (keys beyond it are never needed)
-    const int last = min(p0 + min(tb + QB, a.T) - 1, a.max_seq - 1);
-
-    // Q as the A operand: row lr, dims 16t + 4kq .. +3
-    f32x4v qa[NT];
-    {
-        const int t = min(qw0 + lr, a.T - 1);
-        const float* q = a.qkv + (size_t)t * a.ldqkv + (size_t)h * HD + 4 * kq;
+    // longest tiles first; with heads in multiples of 8 an XCD (workgroup id
+    // mod 8) takes consecutive heads, whose K and V share its L2
+    const int H = a.num_heads, nq = (a.T + 31) / 32, id = (int)blockIdx.x;
+    const int hx = H % 8 == 0 ? H / 8 : H, j = H % 8 == 0 ? id >> 3 : id;
+    const int head = (H % 8 == 0 ? (id & 7) * hx : 0) + j % hx, t0 = (nq - 1 - j / hx) * 32;
+    AttnWave<HD> w;
+    w.init(a, head, t0, lane);
+    float4 kf[2 * NS];
+    vecT vf[16];
+    // half `part` of a block's K dims or V keys; the loads are kept where they
+    // are written (the registers of both whole blocks do not fit two waves per SIMD)
+    auto load_k = [&](int k0, int part) {
+        const float* row = w.kbase + (size_t)min(k0 + w.r32, w.last) * w.kvd + 4 * w.h;
 #pragma unroll
-        for (int t4 = 0; t4 < NT; ++t4) qa[t4] = *reinterpret_cast<const f32x4v*>(q + 16 * t4);
+        for (int i = part * NS; i < (part + 1) * NS; ++i) kf[i] = *reinterpret_cast<const float4*>(row + 8 * i);
+        asm volatile("" ::: "memory");
+    };
+    auto load_v = [&](int k0, int part) {
+#pragma unroll
+        for (int v = 8 * part; v < 8 * part + 8; ++v)
+            vf[v] = *reinterpret_cast<const vecT*>(
+                w.vbase + (size_t)min(k0 + 8 * (v >> 2) + 4 * w.h + (v & 3), w.last) * w.kvd + NT * w.r32);
+        asm volatile("" ::: "memory");
+    };
+    if (wave < w.nblk) {
+        load_k(32 * wave, 0);
+        load_k(32 * wave, 1);
     }
-    // this lane's output rows: queries qw0 + 4kq + i
-    int qpos[4];
-    bool qlive[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int t = qw0 + 4 * kq + i;
-        qlive[i] = t < a.T;
-        qpos[i] = min(p0 + t, a.max_seq - 1);
+    for (int s = wave; s < NS; s += 4) {
+        const Split8 q = w.query(s);
+        sQ[(0 * NS + s) * 64 + lane] = q.h;
+        sQ[(1 * NS + s) * 64 + lane] = q.m;
+        sQ[(2 * NS + s) * 64 + lane] = q.l;
     }
-    float m[4], l[4];
-    f32x4v acc[NT];
+    __syncthreads();
+    float odd = 0.f;
+    for (int b = wave; b < w.nblk; b += 4) {
+        const int k0 = 32 * b;
+        load_v(k0, 0);
+        f32x16v s;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        m[i] = -INFINITY;
-        l[i] = 0.f;
-    }
+        for (int v = 0; v < 16; ++v) s[v] = 0.f;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    const int wlast = min(p0 + min(qw0 + QW, a.T) - 1, a.max_seq - 1);  // this wave's last
-
-    for (int k0 = 0; k0 <= last; k0 += KB) {
-        __syncthreads();  // the previous block's sK / sVt consumed
-        // K rows: thread -> (key r, 4 dims c); V: (key r fastest) -> sVt[dims][r]
-        for (int e = tid; e < KB * HD / 4; e += 256) {
-            const int r = e / (HD / 4), c = (e - r * (HD / 4)) * 4;
-            const int kp = min(k0 + r, last);
-            *reinterpret_cast<float4*>(&sK[r][c]) = *reinterpret_cast<const float4*>(
-                a.kcache + (size_t)kp * a.kvd + (size_t)kvh * HD + c);
-            const int rv = e % KB, cv = (e / KB) * 4;
-            const int kv = min(k0 + rv, last);
-            const float4 v = *reinterpret_cast<const float4*>(a.vcache + (size_t)kv * a.kvd +
-                                                              (size_t)kvh * HD + cv);
-            sVt[cv + 0][rv] = v.x;
-            sVt[cv + 1][rv] = v.y;
-            sVt[cv + 2][rv] = v.z;
-            sVt[cv + 3][rv] = v.w;
+        for (int i = 0; i < NS; ++i) {
+            const Split8 q{sQ[(0 * NS + i) * 64 + lane], sQ[(1 * NS + i) * 64 + lane],
+                           sQ[(2 * NS + i) * 64 + lane]};
+            mfma_split(split8_rne({kf[2 * i].x, kf[2 * i].y, kf[2 * i].z, kf[2 * i].w, kf[2 * i + 1].x,
+                                   kf[2 * i + 1].y, kf[2 * i + 1].z, kf[2 * i + 1].w}), q, s);
         }
-        __syncthreads();
-        if (k0 > wlast) continue;  // (uniform per wave) keys after every query of the wave
-
-        // S = Q K^T: 2 blocks of 16 keys; lane: key 16nb + lr, queries 4kq + i
-        f32x4v s[2];
+        load_v(k0, 1);
+        load_k(k0 + 128, 0);  // (rows past the last are read again, not used)
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            s[nb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        for (int v = 0; v < 16; ++v) odd = fmaf(s[v], 0.f, odd);
+        w.softmax(k0, s);
 #pragma unroll
-            for (int t4 = 0; t4 < NT; ++t4) {
-                const f32x4v kb = *reinterpret_cast<const f32x4v*>(&sK[16 * nb + lr][16 * t4 + 4 * kq]);
+        for (int k = 0; k < 2; ++k) {
+            const Split8 p = split8_rne({s[8 * k], s[8 * k + 1], s[8 * k + 2], s[8 * k + 3], s[8 * k + 4],
+                                         s[8 * k + 5], s[8 * k + 6], s[8 * k + 7]});
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    s[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[t4][u], kb[u], s[nb], 0, 0, 0);
+            for (int i = 0; i < NT; ++i) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = vf[8 * k + e][i];
+                mfma_split(split8_rne(x), p, w.acc[i]);
             }
-        }
-        // online softmax per query row (the 16 lanes of a kq group hold its keys)
-        float f[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float sv[2];
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                const int kp = k0 + 16 * nb + lr;
-                sv[nb] = (qlive[i] && kp <= qpos[i]) ? s[nb][i] * a.scale : -INFINITY;
-            }
-            float bm = fmaxf(sv[0], sv[1]);
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) bm = fmaxf(bm, __shfl_xor(bm, o));
-            const float mn = fmaxf(m[i], bm);
-            f[i] = m[i] == -INFINITY ? 0.f : expf(m[i] - mn);
-            float ls = 0.f;
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                const float pe = sv[nb] == -INFINITY ? 0.f : expf(sv[nb] - mn);
-                sP[wave][4 * kq + i][16 * nb + lr] = pe;
-                ls += pe;
-            }
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) ls += __shfl_xor(ls, o);
-            l[i] = fmaf(l[i], f[i], ls);
-            m[i] = mn;
-        }
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[j][i] *= f[i];
-        // O += P V: A = P (row lr, keys 16t + 4kq + u), B = V^T rows (dim 16j + lr)
-#pragma unroll
-        for (int t2 = 0; t2 < KB / 16; ++t2) {
-            const f32x4v pa = *reinterpret_cast<const f32x4v*>(&sP[wave][lr][16 * t2 + 4 * kq]);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const f32x4v vb = *reinterpret_cast<const f32x4v*>(&sVt[16 * j + lr][16 * t2 + 4 * kq]);
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[u], vb[u], acc[j], 0, 0, 0);
-            }
+            if (k == 0) load_k(k0 + 128, 1);
         }
     }
-    // lane: dims 16j + lr of queries 4kq + i
+    if (w.not_finite(odd)) w.f32_blocks(wave, 4);
+    // the four waves' partials: out = sum_w acc_w e^(m_w - M) / sum_w l_w e^(m_w - M)
+    const float l = halves_add(w.l);
+    __syncthreads();  // (every wave is done with the queries)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (!qlive[i]) continue;
-        float* out = a.attn + (size_t)(qw0 + 4 * kq + i) * a.qd + (size_t)h * HD;
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) out[16 * j + lr] = acc[j][i] / l[i];
+        for (int v = 0; v < 16; ++v) sO[(wave * 16 * NT + v * NT + i) * 64 + lane] = w.acc[i][v];
+    if (w.h == 0) {
+        s_m[wave][w.r32] = w.m;
+        s_l[wave][w.r32] = l;
+    }
+    __syncthreads();
+    float f[4], M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) M = fmaxf(M, s_m[k][w.r32]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        f[k] = s_m[k][w.r32] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((s_m[k][w.r32] - M) * w.c);
+        L = fmaf(s_l[k][w.r32], f[k], L);
+    }
+    if (t0 + w.r32 >= a.T) return;
+    // wave w: accumulator rows 8 w + 4 h .. + 3 of every tile
+    float* out = a.attn + (size_t)w.t * a.qd + (size_t)head * HD;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        vecT o;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            float x = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                x = fmaf(sO[(k * 16 * NT + (4 * wave + v) * NT + i) * 64 + lane], f[k], x);
+            o[i] = x / L;
+        }
+        *reinterpret_cast<vecT*>(out + NT * (8 * wave + 4 * w.h + v)) = o;
     }
 }
 
 int launch_pf_attention(const PfDenseArgs& a, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid_m((unsigned)a.num_heads, (unsigned)((a.T + 63) / 64));
+    const dim3 grid_s((unsigned)a.num_heads * (unsigned)((a.T + 31) / 32));
     const dim3 grid((unsigned)a.num_heads, (unsigned)((a.T + 15) / 16));
     switch (a.head_dim) {
-        case 64: hipLaunchKernelGGL(attn_mfma_kernel<64>, grid_m, dim3(256), 0, st, a); break;
-        case 128: hipLaunchKernelGGL(attn_mfma_kernel<128>, grid_m, dim3(256), 0, st, a); break;
+        case 64: hipLaunchKernelGGL(attn_split_kernel<64>, grid_s, dim3(256), 0, st, a); break;
+        case 128: hipLaunchKernelGGL(attn_split_kernel<128>, grid_s, dim3(256), 0, st, a); break;
         case 256: hipLaunchKernelGGL(attn_causal_kernel<256>, grid, dim3(256), 0, st, a); break;
         default: return (int)hipErrorInvalidValue;
     }

@@ -60,3 +60,72 @@ def test_rmsnorm_edges(ops_ctx, n):
     assert rel_l2(dout.download(np.float32), orc.rmsnorm(x, w, 1e-5)) < 1e-6
     for b in (dx, dw, dout):
         b.free()
+
+
+# ---- prefill attention ------------------------------------------------------------------
+
+
+def _prefill_matches(p, toks, Ts):
+    """The prompts' last logits against the oracle's token-by-token run: with
+    the MoE block zeroed every operation is an f32 sum, held to 1e-5 as the
+    other dense prefill tests hold it."""
+    off = 0
+    for T in Ts:
+        say(f"prefill T={T} at position {off}")
+        _, g_lg = p.dec.prefill(toks[off:off + T], return_logits=True)
+        for t in toks[off:off + T]:
+            _, w_lg = p.orc.step(int(t))
+        off += T
+        assert np.all(np.isfinite(g_lg))
+        rel = rel_l2(g_lg, w_lg)
+        assert rel < 1e-5, f"T={T}: rel L2 {rel:.2e}"
+
+
+@pytest.mark.parametrize("heads,kv,hd,Ts", [(2, 1, 64, (31,)), (2, 1, 64, (32, 1, 32)),
+                                            (3, 3, 64, (33, 95)), (8, 2, 128, (129,)),
+                                            (16, 4, 128, (64, 3, 127)), (24, 8, 64, (40,))])
+def test_prefill_attention_tile_edges(heads, kv, hd, Ts):
+    """32-query tiles and 32-key blocks one short of, at and past their edges,
+    behind an earlier context too, heads in and not in multiples of 8; two
+    layers, so that every query's output reaches the last logits."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    wl = synth.DecoderWorkload("edges", synth.CONFIGS["tiny_renorm"], 2, 300, heads, kv, hd,
+                               1e4, True, 8, 8)
+    p = Pair(wl, seed=61, max_seq=sum(Ts))
+    try:
+        _zero_experts(p)
+        _prefill_matches(p, synth.prompt_tokens(wl, 3, sum(Ts)), Ts)
+    finally:
+        p.close()
+
+
+def test_prefill_attention_keys_past_the_split():
+    """A K value of 3.397e38 rounds to infinity in bf16 (its parts would add up
+    to NaN): the wave's blocks are multiplied on f32 MFMA instead.  eps 0 and
+    an embedding of ones make the projections' input exactly 1; queries of
+    2e-38 keep the scores below 1."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import _lib, synth
+    wl = synth.DecoderWorkload("huge", synth.CONFIGS["tiny"], 1, 300, 2, 1, 64, 1e4, False, 8, 8,
+                               rms_eps=0.0)
+    p = Pair(wl, seed=62, max_seq=48)
+    try:
+        _zero_experts(p)
+        h, kvd, qd = 128, 64, 128
+        wq, wk = np.zeros((qd, h), np.float32), np.zeros((kvd, h), np.float32)
+        wq[[0, 64], 0] = 2e-38
+        wk[0, 0], wk[0, 1] = 3.3895e38, 8e35
+        new = {(_lib.W_EMBED, "embed"): np.ones((wl.vocab, h)), (_lib.W_IN_NORM, "in_norm"): np.ones(h),
+               (_lib.W_Q, "q"): wq, (_lib.W_K, "k"): wk}
+        for (which, name), a in new.items():
+            bits = bf16(a)
+            p.dec.upload(which, 0, bits)
+            if which in _lib.W_PER_LAYER:
+                p.orc.t[name][0] = bits
+            else:
+                p.orc.t[name] = bits
+        _prefill_matches(p, synth.prompt_tokens(wl, 5, 45), (40, 5))
+        assert float(np.abs(p.orc.kc).max()) > 3.396e38
+    finally:
+        p.close()
