@@ -205,8 +205,11 @@ int32_t m1moe_attention_decode(m1moe_ctx_t ctx, const float* d_q, const float* d
     if (seq_len <= 0 || seq_len > 65536)
         return fail(M1MOE_ERR_INVALID, "seq_len %d out of range [1, 65536]", seq_len);
     if ((rc = set_device(ctx))) return rc;
-    if ((rc = ensure_attn_scratch(ctx, attention_partial_floats(num_heads, head_dim, seq_len)))) return rc;
     AttnArgs a{};
+    a.qh = attention_qh(num_heads / num_kv_heads);
+    a.cus = ctx->cus;
+    a.nch = attention_chunks(seq_len, num_heads / a.qh, a.cus);
+    if ((rc = ensure_attn_scratch(ctx, attention_partial_floats(num_heads, head_dim, a.nch)))) return rc;
     a.fused = 0;
     a.q = d_q;
     a.kcache = const_cast<float*>(d_kcache);  // read only when fused = 0
@@ -221,9 +224,6 @@ int32_t m1moe_attention_decode(m1moe_ctx_t ctx, const float* d_q, const float* d
     a.num_kv_heads = num_kv_heads;
     a.hpkv = num_heads / num_kv_heads;
     a.head_dim = head_dim;
-    a.qh = attention_qh(a.hpkv);
-    a.cus = ctx->cus;
-    a.chunk = attention_chunk(seq_len, num_heads / a.qh, a.cus);
     a.kv_pos = (int64_t)num_kv_heads * head_dim;   // the caller's [seq_len][num_kv_heads][head_dim]
     a.kv_head = head_dim;
     a.scale = 1.0f / sqrtf((float)head_dim);
@@ -283,7 +283,9 @@ int32_t m1moe_dec_create(m1moe_ctx_t moe, const m1moe_dec_shape* s, m1moe_dec_t*
     d->loaded.assign((size_t)kNumW * d->L, false);
     const uint64_t h = d->h, L = d->L, V = s->vocab, qd = d->qd, kvd = d->kvd, hd = s->head_dim;
     const uint64_t ms = s->max_seq;
-    const uint64_t part = (uint64_t)attention_partial_floats(s->num_heads, s->head_dim, s->max_seq);
+    const int32_t groups = s->num_heads / attention_qh(s->num_heads / s->num_kv_heads);
+    const uint64_t part = (uint64_t)attention_partial_floats(
+        s->num_heads, s->head_dim, attention_chunks(s->max_seq, groups, moe->cus));
     if ((rc = dec_alloc(d, (void**)&d->embed, V * h * 2, "embedding")) ||
         (rc = dec_alloc(d, (void**)&d->lm_head, V * h * 2, "lm_head")) ||
         (rc = dec_alloc(d, (void**)&d->final_norm, h * 2, "final norm")) ||
@@ -414,7 +416,7 @@ int32_t dec_step(m1moe_dec_t dec, const int32_t* tok_in, int32_t* tok_out, int32
     at.head_dim = hd;
     at.qh = attention_qh(at.hpkv);
     at.cus = ctx->cus;
-    at.chunk = attention_chunk(dec->sh.max_seq, at.num_heads / at.qh, at.cus);
+    at.nch = attention_chunks(dec->sh.max_seq, at.num_heads / at.qh, at.cus);
     at.kv_pos = kvd;
     at.kv_head = hd;
     at.scale = 1.0f / sqrtf((float)hd);
@@ -472,8 +474,7 @@ int32_t dec_step(m1moe_dec_t dec, const int32_t* tok_in, int32_t* tok_out, int32
         o.attn_heads = at.num_heads;
         o.attn_qh = at.qh;
         o.attn_hd = hd;
-        o.attn_chunk = at.chunk;
-        o.attn_nch = (at.max_seq + at.chunk - 1) / at.chunk;
+        o.attn_nch = at.nch;
         o.pos = dec->pos;
         o.max_seq = at.max_seq;
         if ((rc = launched(launch_matvec_bf16(o, st), "o_proj"))) return rc;

@@ -210,8 +210,8 @@ __device__ __forceinline__ RowRef mv_row(const MvArgs& a, int row) {
 // partials are read once per kv head rather than once per matvec workgroup).
 // The attention launch and the matvec that stages its output both decide
 // with this function.
-__device__ __forceinline__ int attn_defer_nact(int p, int max_seq, int chunk, int num_heads) {
-    const int seq = p < max_seq ? p + 1 : max_seq;
+__device__ __forceinline__ int attn_defer_nact(int p, int max_seq, int nch, int num_heads) {
+    const int seq = p < max_seq ? p + 1 : max_seq, chunk = attn_chunk(seq, nch);
     const int nact = (seq + chunk - 1) / chunk;
     return (nact > 1 && nact <= kAttnDeferChunks && nact * num_heads <= kAttnDeferHeadChunks)
                ? nact
@@ -286,8 +286,8 @@ __device__ void mv_stage(const MvArgs& a, float* s_x, float* s_red) {
             ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
         }
     } else if (a.attn_part &&
-               attn_defer_nact(*a.pos, a.max_seq, a.attn_chunk, a.attn_heads) > 0) {
-        ss = mv_stage_attn(a, attn_defer_nact(*a.pos, a.max_seq, a.attn_chunk, a.attn_heads),
+               attn_defer_nact(*a.pos, a.max_seq, a.attn_nch, a.attn_heads) > 0) {
+        ss = mv_stage_attn(a, attn_defer_nact(*a.pos, a.max_seq, a.attn_nch, a.attn_heads),
                            s_x);
     } else {
         const float4* x4 = reinterpret_cast<const float4*>(a.x);
@@ -420,7 +420,7 @@ __global__ __launch_bounds__(256) void matvec_kernel(MvArgs a) {
     if (ngroups > 1) load(1, nxt);
     if (STAGE) {
         if (early && !(a.attn_part &&
-                       attn_defer_nact(*a.pos, a.max_seq, a.attn_chunk, a.attn_heads) > 0))
+                       attn_defer_nact(*a.pos, a.max_seq, a.attn_nch, a.attn_heads) > 0))
             mv_stage_early<XN>(a, s_x, s_red, xv, nwv);
         else
             mv_stage(a, s_x, s_red);
@@ -590,6 +590,20 @@ __device__ __forceinline__ float lane_stride_sum(float v) {
     return halves_sum(v);
 }
 
+// The maximum over the same lanes.
+__device__ __forceinline__ float swap_max(float v, bool halves) {
+    const uint32_t u = __float_as_uint(v);
+    const auto r = halves ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
+                          : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <int LP>
+__device__ __forceinline__ float lane_stride_max(float v) {
+    if (LP == 8) v = fmaxf(v, dpp_f32<kDppRor8>(v, v));
+    if (LP <= 16) v = swap_max(v, false);
+    return swap_max(v, true);
+}
+
 __device__ __forceinline__ uint32_t ld_coh_u32(const uint32_t* p) {
     return __hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -734,16 +748,22 @@ __device__ void attn_merge_share(const AttnArgs& a, int g, int c, int nch, int n
 
 
 // Workgroup (g, c): q heads g*QH .. g*QH+QH-1 (one kv head), positions
-// c*a.chunk .. (c+1)*a.chunk - 1, walked SCH at a time with a running max
-// and sum (the softmax of attnSoftmax, Shaders.metal:245-289, in pieces).
-// Lanes take 8 dims of one position each (HD/8 lanes per position), so every
-// K or V row is one coalesced read shared by the QH heads.  V: 0 one set of
-// K/V registers, 64-position sub-chunks; 1 two sets (chunks of several
-// sub-chunks); 2 one wide sub-chunk of up to attn_wide_sub<HD>() positions
-// (chunks of 65..kAttnWideChunk positions, so that the grid fits the CUs).
-template <int HD>
-__host__ __device__ constexpr int attn_wide_sub() { return HD == 64 ? 96 : 80; }
-
+// c*chunk .. (c+1)*chunk - 1.  Lanes take 8 dims of one position each (LP =
+// HD/8 lanes per position, 64/LP positions per wave and load), so every K or V
+// row is one coalesced read shared by the QH heads.  Each wave walks
+// batches of SB loads (V 1: batches wave, wave + 4, ... of the chunk, two in
+// flight; V 0 and 2: its quarter of the chunk as one batch of at most 4 or 5
+// loads, no second register set), and each of its 64/LP position groups keeps
+// a running softmax of its own (the softmax of attnSoftmax, Shaders.metal:245-289, in pieces), merged
+// across the wave's lanes and the waves only at the end of the chunk: no
+// barrier and no LDS between the first row and the last.  Bound by HBM at long
+// contexts (2 x kv_heads x head_dim x 4 bytes per position), by the chain
+// launch - rows - merge at short ones.  Against 64-position sub-chunks that all
+// four waves scored, normalised and summed between three barriers: 16 heads of
+// 128 at 200 / 2112 / 8192 positions 7.0 / 13.6 / 33.1 -> 6.7 / 12.2 / 29.7 us,
+// 32 q / 8 kv heads at 2112 / 5003 / 8192 12.0 / 30.6 / 24.7 -> 11.0 / 16.9 /
+// 20.5 us (5003 with its old 320 workgroups of 128 positions on 256 CUs; 41 MB
+// of rows in 16.9 us, 2.4 TB/s launch and merge included).
 // The planes z >= 1 of an attention grid: workgroup p of the P in them
 // (linear dispatch number A + p after the A attention workgroups, so XCD
 // p mod 8 when A and P are multiples of 8)
@@ -773,25 +793,30 @@ __device__ void attn_prefetch(const AttnArgs& a) {
     asm volatile("" ::"v"(acc));
 }
 
+// Loads per batch.  V 0: a quarter of 64 positions; V 2: of 96 (head_dim 64) or
+// 80 (128); V 1: what two register sets leave room for.
 template <int HD, int QH, int V>
-__global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
+__host__ __device__ constexpr int attn_sb() {
+    return V == 0 ? HD / 32 : V == 2 ? HD / 32 + 1 : QH == 8 ? 2 : 4;
+}
+
+template <int HD, int QH, int V>
+__global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
     if (blockIdx.z) {
         attn_prefetch(a);
         return;
     }
-    constexpr bool TWO = V == 1;
-    constexpr int SCH = V == 2 ? attn_wide_sub<HD>() : kAttnChunk;   // positions per sub-chunk
     constexpr int LP = HD / 8;                 // lanes per position
-    constexpr int PPI = 64 / LP;               // positions per wave and iteration
-    constexpr int PW = SCH / 4;                // positions per wave per sub-chunk
-    constexpr int IT = PW / PPI;               // iterations
-    static_assert(PW % PPI == 0 && SCH <= 128, "whole iterations, at most two positions per softmax lane");
+    constexpr int PPI = 64 / LP;               // positions per wave and load
+    constexpr bool TWO = V == 1;
+    constexpr int SB = attn_sb<HD, QH, V>();   // loads per batch
+    constexpr int BP = SB * PPI;               // positions per batch
     constexpr int HALF = HD / 2;
     __shared__ __attribute__((aligned(16))) float s_q[QH][HD];
     __shared__ __attribute__((aligned(16))) float s_kv[2][HD];
-    __shared__ float s_p[QH][SCH];
     __shared__ __attribute__((aligned(16))) float s_acc[4][QH][HD];
-    __shared__ float s_m[QH], s_l[QH], s_f[QH];
+    __shared__ float s_wm[4][QH], s_wl[4][QH];     // per wave: maximum (exponent of two), sum
+    __shared__ float s_l[QH];                      // merge: sum per head
     __shared__ float s_st[2][QH][kAttnMaxChunks];  // merge: chunk max and sum
     __shared__ int s_flag;
     __shared__ uint32_t s_tag;
@@ -829,9 +854,10 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
         seq = a.seq_len;
     }
     const bool has_new = a.fused && p < a.max_seq;  // row p comes from k_new / v_new
-    const int c0 = c * a.chunk, c1 = min(c0 + a.chunk, seq);
-    const int nact = min(nch, (seq + a.chunk - 1) / a.chunk);  // workgroups with positions
-    const bool defer = a.defer && attn_defer_nact(p, a.max_seq, a.chunk, a.num_heads) > 0;
+    const int chunk = attn_chunk(seq, nch);
+    const int c0 = c * chunk, c1 = min(c0 + chunk, seq);
+    const int nact = (seq + chunk - 1) / chunk;  // workgroups with positions
+    const bool defer = a.defer && attn_defer_nact(p, a.max_seq, nch, a.num_heads) > 0;
     const bool sync = a.sync_merge && !defer && attn_sync_fits<HD, QH>(nact);
     float* part = a.partial + ((size_t)g * nch + c) * QH * (HD + 2);
     unsigned long long* part64 =
@@ -839,38 +865,32 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
     if (sync && tid == 0) s_tag = ld_coh_u32(a.gen) + 1u;
 
     if (c0 < seq) {
-        // this lane's K and V rows of a 64-position sub-chunk (row p, not yet
-        // in the cache, comes from LDS once it is prepared)
-        // two sub-chunks of rows in flight (A, B alternate)
+        // this wave's positions: batches of BP from w0, 4 BP apart, below w1
+        const int wpos = TWO ? BP : ((c1 - c0 + PPI - 1) / PPI + 3) / 4 * PPI;
+        const int w0 = c0 + wave * wpos, w1 = TWO ? c1 : min(w0 + wpos, c1);
+        // this lane's K and V rows of a batch (rows past the chunk's last are that
+        // row again, left out below; row p, not yet in the cache, comes from LDS
+        // once it is prepared)
         struct KVRows {
-            float k[IT][8], v[IT][8];
+            float4 k[SB][2], v[SB][2];
         };
         KVRows A, B;
+        const float* kb = a.kcache + (size_t)kvh * a.kv_head + 8 * lp;
+        const float* vb = a.vcache + (size_t)kvh * a.kv_head + 8 * lp;
         auto load_rows = [&](int p0, KVRows& R) {
 #pragma unroll
-            for (int it = 0; it < IT; ++it) {
-                const int pp = p0 + wave * PW + it * PPI + pg;
-                float4 k0 = {0.f, 0.f, 0.f, 0.f}, k1 = k0, v0 = k0, v1 = k0;
-                if (pp < c1 && !(has_new && pp == p)) {
-                    const size_t off = (size_t)pp * a.kv_pos + (size_t)kvh * a.kv_head + 8 * lp;
-                    k0 = *reinterpret_cast<const float4*>(a.kcache + off);
-                    k1 = *reinterpret_cast<const float4*>(a.kcache + off + 4);
-                    v0 = *reinterpret_cast<const float4*>(a.vcache + off);
-                    v1 = *reinterpret_cast<const float4*>(a.vcache + off + 4);
-                }
-                R.k[it][0] = k0.x, R.k[it][1] = k0.y, R.k[it][2] = k0.z, R.k[it][3] = k0.w;
-                R.k[it][4] = k1.x, R.k[it][5] = k1.y, R.k[it][6] = k1.z, R.k[it][7] = k1.w;
-                R.v[it][0] = v0.x, R.v[it][1] = v0.y, R.v[it][2] = v0.z, R.v[it][3] = v0.w;
-                R.v[it][4] = v1.x, R.v[it][5] = v1.y, R.v[it][6] = v1.z, R.v[it][7] = v1.w;
+            for (int it = 0; it < SB; ++it) {
+                const size_t off = (size_t)min(p0 + it * PPI + pg, c1 - 1) * a.kv_pos;
+                R.k[it][0] = *reinterpret_cast<const float4*>(kb + off);
+                R.k[it][1] = *reinterpret_cast<const float4*>(kb + off + 4);
+                R.v[it][0] = *reinterpret_cast<const float4*>(vb + off);
+                R.v[it][1] = *reinterpret_cast<const float4*>(vb + off + 4);
             }
         };
-        // (TWO: chunks of several sub-chunks; head_dim 256 has the registers
-        // for one sub-chunk only)
-        constexpr bool kTwo = TWO && HD <= 128;
-        load_rows(c0, A);
-        if (kTwo && c0 + SCH < c1) load_rows(c0 + SCH, B);
-        // keep both sub-chunks' loads here (the compiler may otherwise sink
-        // the second to its first use, a memory round trip later)
+        load_rows(w0, A);
+        if (TWO) load_rows(w0 + 4 * BP, B);
+        // keep both batches' loads here (the compiler may otherwise sink the
+        // second to its first use, a memory round trip later)
         asm volatile("" ::: "memory");
 
         // q heads (and the new k when this workgroup holds row p): per-head
@@ -946,95 +966,106 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
         for (int i = 0; i < QH; ++i)
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
-        if (tid < QH) {
-            s_m[tid] = -INFINITY;
-            s_l[tid] = 0.f;
+        // running maximum of the scores (exponents of two: the queries are scaled)
+        // and sum of this lane's position group (the same in its LP lanes)
+        const Log2Scale scaled(a.scale);
+#pragma unroll
+        for (int i = 0; i < QH; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qv[i][e] = scaled(qv[i][e]);
+        float m[QH], l[QH];
+#pragma unroll
+        for (int i = 0; i < QH; ++i) {
+            m[i] = -INFINITY;
+            l[i] = 0.f;
         }
-
-        auto sub = [&](int p0, KVRows& R) {
-            if (mine_new && p >= p0 && p < p0 + SCH) {
+        auto batch = [&](int p0, KVRows& R) {
+            if (mine_new && p >= p0 && p < p0 + BP) {   // (uniform)
 #pragma unroll
-                for (int it = 0; it < IT; ++it) {
-                    if (p0 + wave * PW + it * PPI + pg != p) continue;
+                for (int it = 0; it < SB; ++it) {
+                    if (p0 + it * PPI + pg != p) continue;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        R.k[it][e] = s_kv[0][8 * lp + e];
-                        R.v[it][e] = s_kv[1][8 * lp + e];
+                    for (int e = 0; e < 2; ++e) {
+                        R.k[it][e] = *reinterpret_cast<const float4*>(&s_kv[0][8 * lp + 4 * e]);
+                        R.v[it][e] = *reinterpret_cast<const float4*>(&s_kv[1][8 * lp + 4 * e]);
                     }
                 }
             }
             // scores (attnScores, Shaders.metal:209-243)
+            float s[SB][QH];
 #pragma unroll
-            for (int it = 0; it < IT; ++it) {
-                const int pl = wave * PW + it * PPI + pg;
+            for (int it = 0; it < SB; ++it)
 #pragma unroll
                 for (int i = 0; i < QH; ++i) {
-                    float d = 0.f;
+                    const float4 k0 = R.k[it][0], k1 = R.k[it][1];
+                    float d = qv[i][0] * k0.x;
+                    d = fmaf(qv[i][1], k0.y, d);
+                    d = fmaf(qv[i][2], k0.z, d);
+                    d = fmaf(qv[i][3], k0.w, d);
+                    d = fmaf(qv[i][4], k1.x, d);
+                    d = fmaf(qv[i][5], k1.y, d);
+                    d = fmaf(qv[i][6], k1.z, d);
+                    d = fmaf(qv[i][7], k1.w, d);
+                    s[it][i] = lane_group_sum<LP>(d);
+                }
+            if (w1 - p0 < BP) {   // (uniform) positions past the wave's: weight 0 on zeros
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) d = fmaf(qv[i][e], R.k[it][e], d);
-                    d = lane_group_sum<LP>(d);
-                    if (lp == 0) s_p[i][pl] = p0 + pl < c1 ? d * a.scale : -INFINITY;
-                }
+                for (int it = 0; it < SB; ++it)
+                    if (p0 + it * PPI + pg >= w1) {
+                        R.v[it][0] = R.v[it][1] = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int i = 0; i < QH; ++i) s[it][i] = -INFINITY;
+                    }
             }
-            __syncthreads();
-            // running max and sum per head; lane = position of the sub-chunk
-            // (and lane + 64 in a wide one)
-            for (int i = wave; i < QH; i += 4) {
-                constexpr bool W2 = SCH > 64;
-                const float sc = s_p[i][lane];
-                const float sc2 = (W2 && lane + 64 < SCH) ? s_p[i][W2 ? lane + 64 : lane] : -INFINITY;
-                const float m_old = s_m[i];
-                const float m = fmaxf(m_old, wave_max(fmaxf(sc, sc2)));
-                const float e = sc == -INFINITY ? 0.f : expf(sc - m);
-                const float e2 = sc2 == -INFINITY ? 0.f : expf(sc2 - m);
-                const float f = m_old == -INFINITY ? 0.f : expf(m_old - m);
-                const float l = wave_sum(W2 ? e + e2 : e);
-                s_p[i][lane] = e;
-                if (W2 && lane + 64 < SCH) s_p[i][W2 ? lane + 64 : lane] = e2;
-                if (lane == 0) {
-                    s_m[i] = m;
-                    s_l[i] = fmaf(s_l[i], f, l);
-                    s_f[i] = f;
-                }
-            }
-            __syncthreads();
-            // weighted V sum (attnValues, :291-326), earlier sub-chunks rescaled
+            // softmax in pieces and the weighted V sum (attnValues, :291-326)
 #pragma unroll
             for (int i = 0; i < QH; ++i) {
-                const float f = s_f[i];
+                float mn = m[i];
+#pragma unroll
+                for (int it = 0; it < SB; ++it) mn = fmaxf(mn, s[it][i]);
+                const float mc = mn == -INFINITY ? 0.f : mn;
+                const float f = __builtin_amdgcn_exp2f(m[i] - mc);
+                m[i] = mn;
+                l[i] *= f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) acc[i][e] *= f;
-            }
 #pragma unroll
-            for (int it = 0; it < IT; ++it) {
-                const int pl = wave * PW + it * PPI + pg;
-#pragma unroll
-                for (int i = 0; i < QH; ++i) {
-                    const float w = s_p[i][pl];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[i][e] = fmaf(w, R.v[it][e], acc[i][e]);
+                for (int it = 0; it < SB; ++it) {
+                    const float w = __builtin_amdgcn_exp2f(s[it][i] - mc);
+                    const float4 v0 = R.v[it][0], v1 = R.v[it][1];
+                    l[i] += w;
+                    acc[i][0] = fmaf(w, v0.x, acc[i][0]);
+                    acc[i][1] = fmaf(w, v0.y, acc[i][1]);
+                    acc[i][2] = fmaf(w, v0.z, acc[i][2]);
+                    acc[i][3] = fmaf(w, v0.w, acc[i][3]);
+                    acc[i][4] = fmaf(w, v1.x, acc[i][4]);
+                    acc[i][5] = fmaf(w, v1.y, acc[i][5]);
+                    acc[i][6] = fmaf(w, v1.z, acc[i][6]);
+                    acc[i][7] = fmaf(w, v1.w, acc[i][7]);
                 }
             }
-            if (p0 + SCH < c1) __syncthreads();  // s_p is rewritten by the next sub-chunk
         };
-        if (!kTwo) {
-            for (int p0 = c0; p0 < c1; p0 += SCH) {
-                sub(p0, A);
-                if (p0 + SCH < c1) load_rows(p0 + SCH, A);
+        if (TWO) {
+            for (int p0 = w0; p0 < w1; p0 += 8 * BP) {
+                batch(p0, A);
+                if (p0 + 4 * BP >= w1) break;
+                load_rows(p0 + 8 * BP, A);
+                batch(p0 + 4 * BP, B);
+                load_rows(p0 + 12 * BP, B);
             }
+        } else if (w0 < w1) {
+            batch(w0, A);
         }
-        for (int p0 = c0; kTwo && p0 < c1; p0 += 2 * SCH) {
-            sub(p0, A);
-            if (p0 + 2 * SCH < c1) load_rows(p0 + 2 * SCH, A);
-            if (p0 + SCH < c1) {
-                sub(p0 + SCH, B);
-                if (p0 + 3 * SCH < c1) load_rows(p0 + 3 * SCH, B);
-            }
+        // the wave's position groups, then (in LDS) its partial
+#pragma unroll
+        for (int i = 0; i < QH; ++i) {
+            const float M = lane_stride_max<LP>(m[i]);
+            const float f = m[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[i] - M);
+            l[i] = lane_stride_sum<LP>(l[i] * f);
+            m[i] = M;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[i][e] = lane_stride_sum<LP>(acc[i][e] * f);
         }
-#pragma unroll
-        for (int i = 0; i < QH; ++i)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[i][e] = lane_stride_sum<LP>(acc[i][e]);
         if (pg == 0) {
 #pragma unroll
             for (int i = 0; i < QH; ++i) {
@@ -1042,42 +1073,67 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
                     float4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
                 *reinterpret_cast<float4*>(&s_acc[wave][i][8 * lp + 4]) =
                     float4{acc[i][4], acc[i][5], acc[i][6], acc[i][7]};
+                if (lp == 0) {
+                    s_wm[wave][i] = m[i];
+                    s_wl[wave][i] = l[i];
+                }
             }
         }
         __syncthreads();
+        // the four waves' partials of (head i, dim d), and of head i's sum
+        auto head_max = [&](int i) {
+            return fmaxf(fmaxf(s_wm[0][i], s_wm[1][i]), fmaxf(s_wm[2][i], s_wm[3][i]));
+        };
+        auto wave_factor = [&](int w, int i, float M) {
+            return s_wm[w][i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_wm[w][i] - M);
+        };
+        auto head_sum = [&](int i, float M) {
+            float t = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) t = fmaf(s_wl[w][i], wave_factor(w, i, M), t);
+            return t;
+        };
+        auto head_acc = [&](int i, int d, float M) {
+            float t = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) t = fmaf(s_acc[w][i][d], wave_factor(w, i, M), t);
+            return t;
+        };
         if (nact == 1) {
             // the only workgroup with positions: no merge
             for (int t = tid; t < QH * HD; t += 256) {
                 const int i = t / HD, d = t - i * HD;
-                a.out[(size_t)(h0 + i) * HD + d] =
-                    (((s_acc[0][i][d] + s_acc[1][i][d]) + s_acc[2][i][d]) + s_acc[3][i][d]) / s_l[i];
+                const float M = head_max(i);
+                a.out[(size_t)(h0 + i) * HD + d] = head_acc(i, d, M) / head_sum(i, M);
             }
             return;
         }
         // (a deferred merge reads the partials in the next launch: plain stores;
         // the synchronous merge: (launch number, value) pairs)
         const uint32_t tag = s_tag;
+        if (tid >= 256 - QH) {   // (the last wave; the chunk's maximum as an exponent of e)
+            const int i = tid - (256 - QH);
+            const float M = head_max(i), L = head_sum(i, M), Ms = M * 0.693147181f;
+            if (sync) {
+                st_coh_u64(part64 + i * (HD + 2), tagged64(tag, Ms));
+                st_coh_u64(part64 + i * (HD + 2) + 1, tagged64(tag, L));
+            } else if (defer) {
+                part[i * (HD + 2)] = Ms;
+                part[i * (HD + 2) + 1] = L;
+            } else {
+                st_coh(part + i * (HD + 2), Ms);
+                st_coh(part + i * (HD + 2) + 1, L);
+            }
+        }
         for (int t = tid; t < QH * HD; t += 256) {
             const int i = t / HD, d = t - i * HD;
-            const float v = ((s_acc[0][i][d] + s_acc[1][i][d]) + s_acc[2][i][d]) + s_acc[3][i][d];
+            const float v = head_acc(i, d, head_max(i));
             if (sync)
                 st_coh_u64(part64 + i * (HD + 2) + 2 + d, tagged64(tag, v));
             else if (defer)
                 part[i * (HD + 2) + 2 + d] = v;
             else
                 st_coh(part + i * (HD + 2) + 2 + d, v);
-        }
-        if (tid < QH) {
-            if (sync) {
-                st_coh_u64(part64 + tid * (HD + 2), tagged64(tag, s_m[tid]));
-                st_coh_u64(part64 + tid * (HD + 2) + 1, tagged64(tag, s_l[tid]));
-            } else if (defer) {
-                part[tid * (HD + 2)] = s_m[tid];
-                part[tid * (HD + 2) + 1] = s_l[tid];
-            } else {
-                st_coh(part + tid * (HD + 2), s_m[tid]);
-                st_coh(part + tid * (HD + 2) + 1, s_l[tid]);
-            }
         }
     }
     if (nact == 1) return;  // (workgroups past the sequence are not read by the merge)
@@ -1272,9 +1328,16 @@ int launch_mv(const MvArgs& a, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-// The kernel's variant for a chunk of `chunk` positions (attn_kernel's V).
-int attn_variant(int chunk) {
-    return chunk <= kAttnChunk ? 0 : (chunk <= kAttnWideChunk ? 2 : 1);
+// The kernel's V for chunks of at most attn_chunk(max_seq, nch) positions (a
+// launch over fewer positions has no longer ones): one batch per wave where a
+// quarter of the chunk fits it.  Eight heads' registers leave that to head_dim
+// 64 (8 q / 1 kv head of 64, 130 positions: 12.0 us with batches of four loads,
+// 11.1 with two).
+int attn_variant(int head_dim, int qh, int max_seq, int nch) {
+    const int n = attn_chunk(max_seq, nch);
+    if (qh == 8 && head_dim != 64) return 1;
+    if (n <= 64) return 0;
+    return head_dim != 256 && n <= (head_dim == 64 ? 96 : 80) ? 2 : 1;
 }
 
 template <int HD, int V>
@@ -1283,21 +1346,21 @@ int launch_attn_v(const AttnArgs& a, dim3 grid, hipStream_t st) {
         case 1: hipLaunchKernelGGL((attn_kernel<HD, 1, V>), grid, dim3(256), 0, st, a); break;
         case 2: hipLaunchKernelGGL((attn_kernel<HD, 2, V>), grid, dim3(256), 0, st, a); break;
         case 4: hipLaunchKernelGGL((attn_kernel<HD, 4, V>), grid, dim3(256), 0, st, a); break;
-        case 8: hipLaunchKernelGGL((attn_kernel<HD, 8, V>), grid, dim3(256), 0, st, a); break;
+        case 8:
+            if constexpr (V == 1 || HD == 64) {
+                hipLaunchKernelGGL((attn_kernel<HD, 8, V>), grid, dim3(256), 0, st, a);
+                break;
+            }
+            return (int)hipErrorInvalidValue;
         default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();
 }
-
 template <int HD>
-int launch_attn_hd(const AttnArgs& a, dim3 grid, hipStream_t st) {
-    // one-sub-chunk workgroups keep no second set of K/V registers, so two of
-    // them fit on a CU (more than 256 workgroups then run at once)
-    switch (attn_variant(a.chunk)) {
-        case 0: return launch_attn_v<HD, 0>(a, grid, st);
-        case 2: return launch_attn_v<HD, 2>(a, grid, st);
-        default: return launch_attn_v<HD, 1>(a, grid, st);
-    }
+int launch_attn_hd(const AttnArgs& a, int v, dim3 grid, hipStream_t st) {
+    if constexpr (HD != 256)
+        if (v == 2) return launch_attn_v<HD, 2>(a, grid, st);
+    return v == 0 ? launch_attn_v<HD, 0>(a, grid, st) : launch_attn_v<HD, 1>(a, grid, st);
 }
 
 }  // namespace
@@ -1340,38 +1403,19 @@ int attention_qh(int hpkv) {
     return 1;
 }
 
-// The fewest 64-position sub-chunks per workgroup that keep at most
-// kAttnMaxChunks workgroups per group.
-int attention_chunk_min(int max_positions) {
-    const int sub = (max_positions + kAttnChunk - 1) / kAttnChunk;  // 64-position sub-chunks
-    return kAttnChunk * ((sub + kAttnMaxChunks - 1) / kAttnMaxChunks);
+// One workgroup per 64 positions while the grid fits the CUs once; above, the
+// positions shared evenly by as many workgroups as there are CUs (the waves
+// stream their rows without waiting for one another, so a second workgroup
+// on some CUs only unbalances them: 32 q / 8 kv heads, 5003 positions, 30.6 us
+// as 320 workgroups of 128 positions, 16.9 as 256 of 157).
+int attention_chunks(int max_positions, int groups, int cus) {
+    const int n = std::min(kAttnMaxChunks, (max_positions + kAttnChunk - 1) / kAttnChunk);
+    const int per = groups > 0 ? cus / groups : 0;   // workgroups per group on the CUs
+    return (long)groups * n <= cus || per < 1 ? n : std::min(n, per);
 }
 
-// When that grid has more workgroups than the device has CUs: if chunks
-// of at most kAttnWideChunk positions fit the groups on the CUs, those (one
-// wide sub-chunk each: 2113 positions x 8 groups on 256 CUs, 67-position
-// chunks, 12.4 -> ~9.8 us); else, from two workgroups per CU on, one
-// workgroup per CU taking more 64-position sub-chunks (32 q / 8 kv heads of
-// 128, 256 CUs: 19.8 -> 16.1 us at 4096 positions, 34.5 -> 25.7 us at 8192).
-// Between the two (one round and a bit, wide chunks too short) the 64-position
-// chunks stay: 256 workgroups of 66 positions in two sub-chunks measured 14.4
-// against 13.5 us for 264 of 64.
-int attention_chunk(int max_positions, int groups, int cus) {
-    const int c = attention_chunk_min(max_positions);
-    const long wgs = (long)groups * ((max_positions + c - 1) / c);
-    const int per = std::min(kAttnMaxChunks, groups > 0 ? cus / groups : 0);   // chunks per group
-    if (per < 1 || wgs <= cus) return c;
-    const int wide = (max_positions + per - 1) / per;
-    if (c == kAttnChunk && wide <= kAttnWideChunk) return wide;
-    if (wgs < 2L * cus) return c;
-    const int sub = (max_positions + kAttnChunk - 1) / kAttnChunk;
-    return std::max(c, kAttnChunk * ((sub + per - 1) / per));
-}
-
-// (sized for attention_chunk_min, whose chunk count bounds attention_chunk's)
-int attention_partial_floats(int num_heads, int head_dim, int max_positions) {
-    const int chunk = attention_chunk_min(max_positions);
-    return 2 * num_heads * ((max_positions + chunk - 1) / chunk) * (head_dim + 2);
+int attention_partial_floats(int num_heads, int head_dim, int nch) {
+    return 2 * num_heads * nch * (head_dim + 2);
 }
 
 namespace {
@@ -1383,14 +1427,19 @@ int attn_occupancy_v(int qh) {
         case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 1, V>, 256, 0); break;
         case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 2, V>, 256, 0); break;
         case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 4, V>, 256, 0); break;
-        case 8: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 8, V>, 256, 0); break;
+        case 8:
+            if constexpr (V == 1 || HD == 64)
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 8, V>, 256, 0);
+            break;
         default: break;
     }
     return e == hipSuccess ? n : 0;
 }
 template <int HD>
 int attn_occupancy_hd(int qh, int v) {
-    return v == 0 ? attn_occupancy_v<HD, 0>(qh) : (v == 2 ? attn_occupancy_v<HD, 2>(qh) : attn_occupancy_v<HD, 1>(qh));
+    if constexpr (HD != 256)
+        if (v == 2) return attn_occupancy_v<HD, 2>(qh);
+    return v == 0 ? attn_occupancy_v<HD, 0>(qh) : attn_occupancy_v<HD, 1>(qh);
 }
 
 // Workgroups of the attention kernel of (head_dim, qh, variant) one CU
@@ -1402,8 +1451,8 @@ int attn_blocks_per_cu(int hd, int qh, int v) {
     std::atomic<int>& slot = g_attn_occ[hi][qh][v];
     int n = slot.load(std::memory_order_relaxed);
     if (n == 0) {
-        n = hd == 64 ? attn_occupancy_hd<64>(qh, v)
-                     : hd == 128 ? attn_occupancy_hd<128>(qh, v) : attn_occupancy_hd<256>(qh, v);
+        n = hd == 64    ? attn_occupancy_hd<64>(qh, v)
+            : hd == 128 ? attn_occupancy_hd<128>(qh, v) : attn_occupancy_hd<256>(qh, v);
         n = n > 0 ? n : -1;
         slot.store(n, std::memory_order_relaxed);
     }
@@ -1413,14 +1462,15 @@ int attn_blocks_per_cu(int hd, int qh, int v) {
 
 bool attention_grid_fits(const AttnArgs& a) {
     if (a.qh <= 0 || a.qh > 8 || a.cus <= 0) return false;
-    const int64_t grid = (int64_t)(a.num_heads / a.qh) * ((a.max_seq + a.chunk - 1) / a.chunk);
-    return (int64_t)attn_blocks_per_cu(a.head_dim, a.qh, attn_variant(a.chunk)) * a.cus >= grid;
+    const int64_t grid = (int64_t)(a.num_heads / a.qh) * a.nch;
+    const int v = attn_variant(a.head_dim, a.qh, a.max_seq, a.nch);
+    return (int64_t)attn_blocks_per_cu(a.head_dim, a.qh, v) * a.cus >= grid;
 }
 
 int launch_attention(const AttnArgs& a, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (a.qh <= 0 || a.num_heads % a.qh || a.hpkv % a.qh ||
-        a.chunk != attention_chunk(a.max_seq, a.num_heads / a.qh, a.cus))
+        a.nch != attention_chunks(a.max_seq, a.num_heads / a.qh, a.cus))
         return (int)hipErrorInvalidValue;
     if (a.kv_pos <= 0 || a.kv_head <= 0) return (int)hipErrorInvalidValue;
     if (a.sync_merge && !(a.gen && a.fin && attention_grid_fits(a))) return (int)hipErrorInvalidValue;
@@ -1429,13 +1479,14 @@ int launch_attention(const AttnArgs& a, void* stream) {
         return (int)hipErrorInvalidValue;
     // (the prefetch planes only where the attention leaves most CUs idle: on a
     // full grid they compete with it, cfg4 2615 -> 2670 us per token)
-    const unsigned gx = (unsigned)(a.num_heads / a.qh), gy = (unsigned)((a.max_seq + a.chunk - 1) / a.chunk);
+    const unsigned gx = (unsigned)(a.num_heads / a.qh), gy = (unsigned)a.nch;
     const bool pf = a.pf && 2 * (int64_t)gx * gy <= a.cus;
     const dim3 grid(gx, gy, pf ? 1u + (unsigned)kAttnPfPlanes : 1u);
+    const int v = attn_variant(a.head_dim, a.qh, a.max_seq, a.nch);
     switch (a.head_dim) {
-        case 64: return launch_attn_hd<64>(a, grid, st);
-        case 128: return launch_attn_hd<128>(a, grid, st);
-        case 256: return launch_attn_hd<256>(a, grid, st);
+        case 64: return launch_attn_hd<64>(a, v, grid, st);
+        case 128: return launch_attn_hd<128>(a, v, grid, st);
+        case 256: return launch_attn_hd<256>(a, v, grid, st);
         default: return (int)hipErrorInvalidValue;
     }
 }

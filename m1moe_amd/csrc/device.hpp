@@ -423,6 +423,21 @@ struct DecLayout {
     }
 };
 
+// q scale log2(e), rounded once: the factor is kept as hi + lo (rounded to f32
+// alone it would shift every exponent of a softmax by up to 2^-25 of itself).
+// Scores of such queries are exponents of two: e^(scale (q . k) - ...) is the
+// hardware exp2 of a difference.
+struct Log2Scale {
+    float hi, lo;
+    __device__ explicit Log2Scale(float scale) {
+        hi = scale * 1.44269504f;
+        lo = fmaf(scale, 1.44269504f, -hi) + scale * 1.92596299e-8f;
+    }
+    __device__ float operator()(float q) const {   // (an infinite q keeps its sign)
+        return fmaf(q, hi, __builtin_amdgcn_fmed3f(q, -3e38f, 3e38f) * lo);
+    }
+};
+
 // silu(g) = g / (1 + e^-g) (Shaders.metal:148, fast-math there) on the
 // hardware exp2 and reciprocal.
 __device__ __forceinline__ float silu_fast(float g) {

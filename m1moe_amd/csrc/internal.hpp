@@ -307,13 +307,14 @@ struct MvArgs {
     // their merge to this one (attention_defers): attn_part is that launch's
     // partial buffer, the other fields its AttnArgs geometry; null: x given
     const float* attn_part;
-    int32_t attn_heads, attn_qh, attn_hd, attn_chunk, attn_nch;
+    int32_t attn_heads, attn_qh, attn_hd, attn_nch;
 };
 
 // Decode attention of one query position.  Workgroup (g, c): q heads
-// g*qh .. g*qh+qh-1 (one kv head) over positions c*chunk .. (c+1)*chunk - 1
-// (chunk = attention_chunk(max_seq, groups, cus): a multiple of 64 or 65 ..
-// kAttnWideChunk, at most kAttnMaxChunks workgroups per kv head).
+// g*qh .. g*qh+qh-1 (one kv head) over positions c*n .. (c+1)*n - 1, n =
+// attn_chunk(positions, nch) of the launch's own positions (nch =
+// attention_chunks(max_seq, groups, cus) workgroups per group, at most
+// kAttnMaxChunks).
 //   fused = 1: q, k_new, v_new are the raw projections of the current token;
 //     q and k get the per-head RMSNorm (q_norm/k_norm non-null) and RoPE at
 //     p = *pos, the new k/v row is stored at cache row p (flag 32 and no
@@ -339,7 +340,7 @@ struct AttnArgs {
     int32_t seq_len;             // fused = 0
     int32_t max_seq;             // cache rows (fused) / seq_len
     int32_t num_heads, num_kv_heads, hpkv, head_dim, qh;
-    int32_t chunk;               // positions per workgroup
+    int32_t nch;                 // workgroups per group (attention_chunks)
     float scale, rope_theta, eps;
     // fused only: for 2 .. kAttnDeferChunks active chunks and num_heads x chunks
     // <= kAttnDeferHeadChunks, write the partials and leave their merge to the
@@ -368,9 +369,8 @@ struct AttnArgs {
     int32_t pf_units;
 };
 
-constexpr int kAttnChunk = 64;   // positions per attention sub-chunk
+constexpr int kAttnChunk = 64;   // positions per attention workgroup at least
 constexpr int kAttnPfPlanes = 1;  // prefetch planes of an attention grid (AttnArgs::pf)
-constexpr int kAttnWideChunk = 80;   // chunks of 65 .. this many positions: one wide sub-chunk
 constexpr int kAttnMaxQH = 8;    // q heads per attention workgroup
 constexpr int kAttnMaxChunks = 64;   // workgroups per kv head
 constexpr int kAttnDeferChunks = 8;        // deferred merge: at most this many chunks
@@ -442,10 +442,16 @@ int matvec_rows_per_workgroup(int rows);
 int launch_matvec_bf16(const MvArgs& a, void* stream);
 // q heads per attention workgroup (0: unsupported hpkv).
 int attention_qh(int hpkv);
-// Positions per attention workgroup for a cache of max_positions, groups
-// (num_heads / qh) workgroups per chunk and cus compute units: a multiple of
-// 64, or 65 .. kAttnWideChunk; at most kAttnMaxChunks chunks.
-int attention_chunk(int max_positions, int groups, int cus);
+// Attention workgroups per group for a cache of max_positions, groups
+// (num_heads / qh) and cus compute units: one per kAttnChunk positions while
+// they fit the CUs, then as many as fill the CUs once; at most kAttnMaxChunks.
+int attention_chunks(int max_positions, int groups, int cus);
+// Positions per workgroup of a launch over `positions` with nch workgroups per
+// group.
+M1MOE_HD inline int attn_chunk(int positions, int nch) {
+    const int n = (positions + nch - 1) / nch;
+    return n > kAttnChunk ? n : kAttnChunk;
+}
 // The whole attention grid of `a` fits on the device at once (a.cus CUs, the
 // occupancy of the kernel instance it launches): the synchronous merge may
 // be used.
@@ -455,7 +461,7 @@ int launch_rope_table(float* table, int max_seq, int head_dim, float theta, void
 constexpr int32_t kAttnSpinLimit = 1 << 20;  // bounded waits of the synchronous merge (~1 s)
 constexpr int kCountWords = 32 * 9;   // a two-level completion counter (dense.hip count_out)
 // floats of the partials buffer (room for the u64 pairs of the synchronous merge)
-int attention_partial_floats(int num_heads, int head_dim, int max_positions);
+int attention_partial_floats(int num_heads, int head_dim, int nch);
 int launch_attention(const AttnArgs& a, void* stream);
 // Greedy token of x[0..n) to *out (ties to the lower index; x[0] NaN gives 0).
 int launch_argmax(const float* x, int n, int32_t* out, void* stream);

@@ -620,7 +620,7 @@ struct AttnWave {
     typedef float vecT __attribute__((ext_vector_type(NT)));
     const float *qrow, *kbase, *vbase;   // the lane's query; the kv head's columns
     int kvd, r32, h, t, qpos, first, last, nblk;
-    float c, m, l;                       // c = scale log2(e); m the running maximum of the raw scores
+    float scale, m, l;                   // m: the running maximum, in exponents of two
     f32x16v acc[NT];
 
     __device__ __forceinline__ void init(const PfDenseArgs& a, int head, int t0, int lane) {
@@ -628,7 +628,7 @@ struct AttnWave {
         r32 = lane & 31;
         h = lane >> 5;
         kvd = a.kvd;
-        c = a.scale * 1.44269504088896341f;
+        scale = a.scale;
         t = min(t0 + r32, a.T - 1);
         qpos = min(p0 + t, a.max_seq - 1);
         first = min(p0 + t0, a.max_seq - 1);                       // the tile's first and
@@ -647,16 +647,16 @@ struct AttnWave {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
     }
-    // k-step s of the lane's query, split
+    // k-step s of the lane's query, scaled (Log2Scale) and split
     __device__ __forceinline__ Split8 query(int s) const {
+        const Log2Scale c(scale);
         const float4 x0 = *reinterpret_cast<const float4*>(qrow + 16 * s + 4 * h);
         const float4 x1 = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 + 4 * h);
-        return split8_rne({x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w});
+        return split8_rne({c(x0.x), c(x0.y), c(x0.z), c(x0.w), c(x1.x), c(x1.y), c(x1.z), c(x1.w)});
     }
     // The running softmax (Shaders.metal:245-289 in pieces) over the lane's 16
-    // keys and the other half's: s becomes the numerators, acc is rescaled.  m
-    // is the largest raw score; e^((s - m) scale) = 2^(s c - m c), c = scale
-    // log2(e), one fused multiply-add (one rounding) and the hardware exp2.
+    // keys and the other half's: s (scores as exponents of two) becomes the
+    // numerators, acc is rescaled.
     __device__ __forceinline__ void softmax(int k0, f32x16v& s) {
         if (k0 + 31 > first) {   // (uniform) some query of the tile does not see the whole block
 #pragma unroll
@@ -667,12 +667,12 @@ struct AttnWave {
 #pragma unroll
         for (int v = 0; v < 16; ++v) bm = fmaxf(bm, s[v]);
         const float mn = fmaxf(m, halves_max(bm));
-        const float mc = mn == -INFINITY ? 0.f : mn * c;   // (no key seen yet: every numerator 0)
-        const float f = __builtin_amdgcn_exp2f(fmaf(m, c, -mc));
+        const float mc = mn == -INFINITY ? 0.f : mn;   // (no key seen yet: every numerator 0)
+        const float f = __builtin_amdgcn_exp2f(m - mc);
         float ls = 0.f;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            s[v] = __builtin_amdgcn_exp2f(fmaf(s[v], c, -mc));
+            s[v] = __builtin_amdgcn_exp2f(s[v] - mc);
             ls += s[v];
         }
         l = fmaf(l, f, ls);
@@ -707,10 +707,11 @@ struct AttnWave {
                 const float4 q = *reinterpret_cast<const float4*>(qrow + 8 * j + 4 * h);
                 const float4 k = *reinterpret_cast<const float4*>(
                     kbase + (size_t)min(k0 + r32, last) * kvd + 8 * j + 4 * h);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.x, q.x, s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.y, q.y, s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.z, q.z, s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.w, q.w, s, 0, 0, 0);
+                const Log2Scale c(scale);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.x, c(q.x), s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.y, c(q.y), s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.z, c(q.z), s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k.w, c(q.w), s, 0, 0, 0);
             }
             softmax(k0, s);
 #pragma unroll
@@ -838,7 +839,7 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(PfDenseArgs a) {
     for (int k = 0; k < 4; ++k) M = fmaxf(M, s_m[k][w.r32]);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        f[k] = s_m[k][w.r32] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((s_m[k][w.r32] - M) * w.c);
+        f[k] = s_m[k][w.r32] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[k][w.r32] - M);
         L = fmaf(s_l[k][w.r32], f[k], L);
     }
     if (t0 + w.r32 >= a.T) return;

@@ -62,6 +62,63 @@ def test_rmsnorm_edges(ops_ctx, n):
         b.free()
 
 
+# ---- decode attention -------------------------------------------------------------------
+
+
+@pytest.mark.parametrize("nh,nkv,hd,sl", [
+    # 64 groups on 256 CUs: four workgroups each, chunks of 64 (one batch per wave),
+    # 65 .. 96 or 80 (one larger batch) and above (two batches in flight)
+    (64, 64, 64, 256), (64, 64, 64, 257), (64, 64, 64, 384), (64, 64, 64, 385),
+    (64, 64, 128, 255), (64, 64, 128, 320), (64, 64, 128, 321), (64, 64, 256, 256),
+    (64, 64, 256, 259), (64, 8, 64, 2049), (64, 8, 128, 130), (64, 8, 128, 8191),
+    # one position past a chunk, past a wave's batch; more groups than CUs
+    (32, 8, 128, 65), (32, 8, 128, 17), (24, 8, 64, 9), (300, 300, 64, 333), (2, 2, 256, 2)])
+def test_attention_decode_chunk_edges(ops_ctx, nh, nkv, hd, sl):
+    """f32 sums of at most 8191 terms against the oracle's f64: 1e-6 (2e-7
+    seen), for lengths around every batch and chunk rule; the last V row is
+    large, so a position read twice or left out shows."""
+    ctx, ops = ops_ctx
+    rng = np.random.default_rng(nh * 7 + sl)
+    kvd = nkv * hd
+    q = rng.normal(0, 1, nh * hd).astype(np.float32)
+    kc = rng.normal(0, 1, (sl, kvd)).astype(np.float32)
+    vc = rng.normal(0, 1, (sl, kvd)).astype(np.float32)
+    vc[-1] *= 100
+    dq, dk, dv, dout = ctx.to_device(q), ctx.to_device(kc), ctx.to_device(vc), ctx.alloc(4 * nh * hd)
+    say(f"attention nh={nh} nkv={nkv} hd={hd} seq={sl}")
+    ops.attention_decode(dq, dk, dv, dout, nh, nkv, hd, sl)
+    ctx.sync()
+    assert rel_l2(dout.download(np.float32), orc.attention(q, kc, vc, nh, nkv, hd, sl)) < 1e-6
+    for b in (dq, dk, dv, dout):
+        b.free()
+
+
+def test_decoder_steps_in_a_long_cache():
+    """A cache of 5000 positions shared by 16 workgroups per head: the chunk
+    grows with the position (64 up to 1024 positions, then more), the
+    deferred, the synchronous and the single-chunk forms in turn."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    wl = synth.DecoderWorkload("longcache", synth.CONFIGS["tiny_renorm"], 1, 300, 16, 16, 64,
+                               1e4, True, 8, 8)
+    p = Pair(wl, seed=63, max_seq=5000)
+    try:
+        _zero_experts(p)
+        toks = synth.prompt_tokens(wl, 7, 1100)
+        off = 0
+        for n, steps in ((60, 8), (190, 4), (800, 3), (20, 3)):
+            _prefill_matches(p, toks[off:], (n,))
+            off += n
+            for t in toks[off:off + steps]:
+                say(f"step at position {off}")
+                _, g_lg = p.dec.forward(int(t), return_logits=True)
+                _, w_lg = p.orc.step(int(t))
+                assert rel_l2(g_lg, w_lg) < 1e-5
+            off += steps
+    finally:
+        p.close()
+
+
 # ---- prefill attention ------------------------------------------------------------------
 
 
