@@ -8,6 +8,7 @@
 // position in device memory (so a greedy loop can be graph-captured).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -94,7 +95,9 @@ struct m1moe_dec {
     float *logits = nullptr, *part = nullptr;
     // prefill scratch for up to pf_cap tokens (grown on demand)
     int32_t pf_cap = 0;
-    float *pf_res = nullptr, *pf_res2 = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr, *pf_attn = nullptr;
+    float *pf_res = nullptr, *pf_res2 = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr;
+    uint16_t* pf_parts = nullptr;  // GEMM inputs as three bf16 parts, [3][T][max(h, qd)]: the normed
+                                   // rows, then the attention output
     float* pf_part = nullptr;  // split-K partials of the prefill GEMMs (kGemmPartFloats)
     uint32_t* cnt = nullptr;   // [dec_cnt_words]: (unused) x 2, attention groups, the
                                // attention's launch number, then (dec_fin_offset) its
@@ -250,7 +253,7 @@ void m1moe_dec_destroy(m1moe_dec_t dec) {
     (void)hipSetDevice(dec->device);
     for (void* p : dec->allocs) (void)hipFree(p);
     for (void* p : {(void*)dec->pf_res, (void*)dec->pf_res2, (void*)dec->pf_xn, (void*)dec->pf_qkv,
-                    (void*)dec->pf_attn, (void*)dec->pf_part})
+                    (void*)dec->pf_parts, (void*)dec->pf_part})
         if (p) (void)hipFree(p);
     delete dec;
 }
@@ -566,7 +569,9 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
         if ((rc = refuse_growth_in_capture(ctx->stream, "the decoder prefill scratch"))) return rc;
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         if (dec->pf_cap > 0) ++ctx->scratch_gen;  // earlier graphs hold the old buffers
-        for (float** b : {&dec->pf_res, &dec->pf_res2, &dec->pf_xn, &dec->pf_qkv, &dec->pf_attn, &dec->pf_part}) {
+        if (dec->pf_parts) (void)hipFree(dec->pf_parts);
+        dec->pf_parts = nullptr;
+        for (float** b : {&dec->pf_res, &dec->pf_res2, &dec->pf_xn, &dec->pf_qkv, &dec->pf_part}) {
             if (*b) (void)hipFree(*b);
             *b = nullptr;
         }
@@ -576,7 +581,7 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
             (rc = device_alloc((void**)&dec->pf_res2, t * h * 4, "prefill residual 2")) ||
             (rc = device_alloc((void**)&dec->pf_xn, t * h * 4, "prefill normed rows")) ||
             (rc = device_alloc((void**)&dec->pf_qkv, t * N * 4, "prefill q/k/v")) ||
-            (rc = device_alloc((void**)&dec->pf_attn, t * qd * 4, "prefill attention")) ||
+            (rc = device_alloc((void**)&dec->pf_parts, t * std::max(h, qd) * 6, "prefill GEMM inputs")) ||
             (rc = device_alloc((void**)&dec->pf_part, kGemmPartFloats * 4, "prefill split-K partials")))
             return rc;
         dec->pf_cap = T;
@@ -589,7 +594,8 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
     a.embed = dec->embed;
     a.res = dec->pf_res;
     a.qkv = dec->pf_qkv;
-    a.attn = dec->pf_attn;
+    a.attn = dec->pf_parts;
+    a.attn_plane = (int64_t)T * qd;
     a.pos = dec->pos;
     a.err = ctx->err;
     a.T = T;
@@ -606,58 +612,30 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
     a.scale = 1.0f / sqrtf((float)hd);
     a.rope_theta = dec->sh.rope_theta;
     a.eps = eps;
-    auto gemm = [&](const float* A, int lda, const uint16_t* W, const float* R, float* C, int ldc, int n,
-                    int k, const char* what) {
-        GemmArgs g{};
-        g.A = A;
-        g.lda = lda;
-        g.W = W;
-        g.R = R;
-        g.C = C;
-        g.ldc = ldc;
-        g.M = T;
-        g.N = n;
-        g.K = k;
-        g.part = dec->pf_part;
-        return launched(launch_gemm(g, st), what);
-    };
-    // q, k and v: one launch over the three weight segments when the prompt
-    // is short (each alone would leave most CUs idle), three launches else
-    const bool merge_qkv = h % 64 == 0 && (long)((N + 127) / 128) * ((T + 127) / 128) < 256;
+    // q, k and v of layer l: one launch over the three weight segments
     auto qkv_gemm = [&](int l) -> int32_t {
-        const uint16_t* wq = dec->wq + (size_t)l * qd * h;
-        const uint16_t* wk = dec->wk + (size_t)l * kvd * h;
-        const uint16_t* wv = dec->wv + (size_t)l * kvd * h;
-        if (merge_qkv) {
-            GemmArgs g{};
-            g.A = dec->pf_xn;
-            g.lda = h;
-            g.W = wq;
-            g.W1 = wk;
-            g.W2 = wv;
-            g.n1 = qd;
-            g.n2 = qd + kvd;
-            g.C = dec->pf_qkv;
-            g.ldc = N;
-            g.M = T;
-            g.N = N;
-            g.K = h;
-            g.part = dec->pf_part;
-            return launched(launch_gemm(g, st), "prefill q/k/v");
-        }
-        int32_t r;
-        if ((r = gemm(dec->pf_xn, h, wq, nullptr, dec->pf_qkv, N, qd, h, "prefill q")) ||
-            (r = gemm(dec->pf_xn, h, wk, nullptr, dec->pf_qkv + qd, N, kvd, h, "prefill k")) ||
-            (r = gemm(dec->pf_xn, h, wv, nullptr, dec->pf_qkv + qd + kvd, N, kvd, h, "prefill v")))
-            return r;
-        return M1MOE_OK;
+        GemmArgs g{};
+        g.X = dec->pf_parts;
+        g.xplane = (int64_t)T * h;
+        g.W = dec->wq + (size_t)l * qd * h;
+        g.W1 = dec->wk + (size_t)l * kvd * h;
+        g.W2 = dec->wv + (size_t)l * kvd * h;
+        g.n1 = qd;
+        g.n2 = qd + kvd;
+        g.C = dec->pf_qkv;
+        g.ldc = N;
+        g.M = T;
+        g.N = N;
+        g.K = h;
+        g.part = dec->pf_part;
+        return launched(launch_gemm(g, st), "prefill q/k/v");
     };
     if ((rc = launched(launch_pf_embed(a, st), "prefill embedding"))) return rc;  // :129-131
     const uint64_t cache_layer = (uint64_t)dec->sh.max_seq * kvd;
     for (int l = 0; l < dec->L; ++l) {
         // input RMSNorm, q/k/v for all T tokens (InferenceEngine.swift:177-192)
-        if ((rc = launched(launch_rmsnorm_rows(dec->pf_res, dec->in_norm + (size_t)l * h, dec->pf_xn, T, h,
-                                               eps, st),
+        if ((rc = launched(launch_rmsnorm_rows(dec->pf_res, dec->in_norm + (size_t)l * h, nullptr, dec->pf_parts,
+                                               (int64_t)T * h, T, h, eps, st),
                            "prefill input norm")) ||
             (rc = qkv_gemm(l)))
             return rc;
@@ -672,8 +650,8 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
         // o_proj + residual (:227-233), post-attention RMSNorm (:234-236)
         // (the norm is made by the GEMM's split-K sum when it has one)
         GemmArgs o{};
-        o.A = dec->pf_attn;
-        o.lda = qd;
+        o.X = dec->pf_parts;
+        o.xplane = (int64_t)T * qd;
         o.W = dec->wo + (size_t)l * h * qd;
         o.R = dec->pf_res;
         o.C = dec->pf_res2;

@@ -444,6 +444,51 @@ __device__ __forceinline__ float silu_fast(float g) {
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896341f));
 }
 
+// vmcnt(n) alone (expcnt and lgkmcnt at their maxima, no wait on them).
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(N >= 0 && N < 64, "vmcnt field is 6 bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// global -> LDS copy of 16 (or 4) bytes per lane from sbase + voff (sbase in
+// SGPRs, voff the lane's 32-bit offset): lane j's bytes land at LDS byte
+// address lds + 16 j (4 j); lds is the same for the whole wave.  Written as
+// inline assembly: the compiler, which cannot tell the ring slots apart,
+// would otherwise wait for every copy in flight before each LDS read.  The
+// kernel waits for the copies itself (vmcnt, which counts them in issue
+// order with every other load) before the barrier that publishes a slot; the
+// compiler's own vmcnt waits for its loads stay safe, as copies it does not
+// know of only make them wait longer.  M0 is not listed as clobbered (the
+// compiler reserves it and warns): these kernels contain no instruction of
+// the compiler's that reads M0 (no LDS-DMA builtins, indexed lane reads or
+// messages; the generated code sets M0 only in these statements).
+__device__ __forceinline__ void lds_copy16(uint32_t voff, const uint8_t* sbase, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff), "s"(sbase), "s"(lds)
+                 : "memory");
+}
+// The same, coherent across the XCDs (sc1: the line is read from memory, not
+// from this XCD's L2): the down GEMM's B when act_fix rewrote act in this launch.
+__device__ __forceinline__ void lds_copy16_coh(uint32_t voff, const uint8_t* sbase, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 sc1"
+                 :
+                 : "v"(voff), "s"(sbase), "s"(lds)
+                 : "memory");
+}
+__device__ __forceinline__ void lds_copy4(uint32_t voff, const uint8_t* sbase, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :
+                 : "v"(voff), "s"(sbase), "s"(lds)
+                 : "memory");
+}
+
+// LDS byte address of a pointer into LDS.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
 __device__ __forceinline__ void flag_error(uint32_t* err, uint32_t code) {
     if (err) atomicOr(err, code);
 }

@@ -379,11 +379,13 @@ constexpr int kMvStageMax = 8192;   // largest staged (normalised / embedded) in
 
 // ---- decoder prefill (prefill_dense.hip) ----
 
-// C[M][N] = A[M][K] W[N][K]^T (+ R[M][N]); A f32 (row stride lda, lda % 4 ==
-// 0), W bf16 row-major, C and R with row stride ldc; K % 32 == 0.
+// C[M][N] = X[M][K] W[N][K]^T (+ R[M][N]); X f32 as three bf16 parts that add
+// up to it, part p at X + p * xplane, rows of K (the producers' store_parts in
+// prefill_dense.hip); W bf16 row-major, C and R with row stride ldc; K % 64 ==
+// 0, N % 4 == 0, ldc % 4 == 0, C and R 16-byte aligned.
 struct GemmArgs {
-    const float* A;
-    int32_t lda;
+    const uint16_t* X;
+    int64_t xplane;              // values between the parts
     const uint16_t* W;
     const float* R;
     float* C;
@@ -395,7 +397,7 @@ struct GemmArgs {
     int32_t splits;              // set by launch_gemm
     // optional second and third weight segments: rows [n1, n2) are rows
     // 0 .. of W1, rows [n2, N) rows 0 .. of W2 (q, k and v in one launch);
-    // null W1: every row from W.  Needs K % 64 == 0.
+    // null W1: every row from W.  n1 and n2 are multiples of 64.
     const uint16_t* W1;
     const uint16_t* W2;
     int32_t n1, n2;
@@ -414,7 +416,8 @@ struct PfDenseArgs {
     const uint16_t* embed;       // [vocab][h]
     float* res;                  // [T][h] residual stream
     float* qkv;                  // [T][ldqkv]: q | k | v
-    float* attn;                 // [T][qd]
+    uint16_t* attn;              // output: three bf16 parts (GemmArgs::X), each [T][qd]
+    int64_t attn_plane;          // values between the parts
     const uint16_t* q_norm;      // [head_dim] or null
     const uint16_t* k_norm;
     float* kcache;               // this layer's [max_seq][kvd]
@@ -427,8 +430,10 @@ struct PfDenseArgs {
 };
 
 int launch_pf_embed(const PfDenseArgs& a, void* stream);
-int launch_rmsnorm_rows(const float* x, const uint16_t* w, float* out, int rows, int n, float eps,
-                        void* stream);
+// RMSNorm of rows of n <= 8192 values (n % 4 == 0), to out (f32) or, parts
+// non-null, to the three parts of a GEMM's input.
+int launch_rmsnorm_rows(const float* x, const uint16_t* w, float* out, uint16_t* parts, int64_t plane, int rows,
+                        int n, float eps, void* stream);
 int launch_gemm(const GemmArgs& g, void* stream);
 int launch_pf_rope_kv(const PfDenseArgs& a, void* stream);
 int launch_pf_attention(const PfDenseArgs& a, void* stream);

@@ -8,13 +8,12 @@
 //   embed_rows     the token rows of the bf16 embedding -> f32 [T][h]
 //                  (InferenceEngine.swift:482-488)
 //   rmsnorm_rows   x * rsqrt(mean(x^2) + eps) * w per row (Shaders.metal:96-134)
-//   gemm_bf3       Y[T][N] = X[T][K] W[N][K]^T (+ R): f32 activations split
-//                  exactly into three bf16 parts, each multiplied with the
-//                  bf16 weights on v_mfma_f32_32x32x16_bf16 (exact products,
-//                  f32 accumulation: the arithmetic of matvecBF16,
-//                  Shaders.metal:328-358, in another order); gemm_kernel does
-//                  the same on v_mfma_f32_16x16x4f32 for a K that is not a
-//                  multiple of 64
+//   gemm_parts     Y[T][N] = X[T][K] W[N][K]^T (+ R): f32 activations, split
+//                  exactly into three bf16 parts by the kernel that produces
+//                  them, each part multiplied with the bf16 weights on
+//                  v_mfma_f32_32x32x16_bf16 (exact products, f32
+//                  accumulation: the arithmetic of matvecBF16,
+//                  Shaders.metal:328-358, in another order)
 //   rope_kv_rows   per token and head: the per-head q/k RMSNorm and RoPE at
 //                  the token's position (InferenceEngine.swift:521-548), k and
 //                  v rows into the caches (:215-220)
@@ -26,6 +25,8 @@
 //
 // The MoE block runs through the grouped prefill (prefill.hip).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "device.hpp"
 #include "internal.hpp"
@@ -49,91 +50,72 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(PfDenseArgs a) {
     for (int d = threadIdx.x; d < a.h; d += 256) out[d] = bf16_to_f32(row[d]);
 }
 
-// One workgroup per row: out = x * rsqrt(sum(x^2) / n + eps) * w.
-__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* x, const uint16_t* w,
-                                                           float* out, int n, float eps) {
+// The three bf16 parts of a GEMM's f32 input, made by the kernel that produces
+// it (row norms, attention): plane p of [3][T][n] holds part p of every value.
+// hi = x with the low 16 bits cleared, mid = the same of x - hi, lo = x - hi -
+// mid: 24 significant bits = 8 + 8 + 8, so the parts add up to x exactly.
+// N = 4 or 2 consecutive values at `at`.
+template <int N>
+__device__ __forceinline__ void store_parts(uint16_t* at, int64_t plane, const float (&x)[N]) {
+    uint32_t h[N], m[N], l[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        h[i] = __float_as_uint(x[i]) & 0xffff0000u;
+        const float r = x[i] - __uint_as_float(h[i]);
+        m[i] = __float_as_uint(r) & 0xffff0000u;
+        l[i] = __float_as_uint(r - __uint_as_float(m[i]));
+    }
+    auto put = [&](uint16_t* p, const uint32_t (&v)[N]) {
+        if constexpr (N == 4)
+            *reinterpret_cast<uint2*>(p) = make_uint2(v[0] >> 16 | (v[1] & 0xffff0000u),
+                                                      v[2] >> 16 | (v[3] & 0xffff0000u));
+        else
+            *reinterpret_cast<uint32_t*>(p) = v[0] >> 16 | (v[1] & 0xffff0000u);
+    };
+    put(at, h);
+    put(at + plane, m);
+    put(at + 2 * plane, l);
+}
+
+// One workgroup per row: out = x * rsqrt(sum(x^2) / n + eps) * w, as f32 (out)
+// or as the three parts of a GEMM's input (parts, rows of n).  n % 4 == 0, n <=
+// 1024 NV: a thread keeps its NV groups of four in registers, so x is read
+// once (2048 rows of 4096: 18.0 -> 13.0 us).
+template <int NV>
+__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* x, const uint16_t* w, float* out,
+                                                           uint16_t* parts, int64_t plane, int n, float eps) {
     __shared__ float s_red[4];
-    const float* xr = x + (size_t)blockIdx.x * n;
-    float* o = out + (size_t)blockIdx.x * n;
+    const size_t row = (size_t)blockIdx.x * n;
+    const int tid = threadIdx.x, n4 = n >> 2;
+    float4 v[NV];
+    uint2 b[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = min(tid + 256 * j, n4 - 1);
+        v[j] = reinterpret_cast<const float4*>(x + row)[i];
+        b[j] = reinterpret_cast<const uint2*>(w)[i];
+    }
     float acc = 0.f;
-    for (int i = threadIdx.x; i < n; i += 256) acc = fmaf(xr[i], xr[i], acc);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+        if (tid + 256 * j < n4)
+            acc = fmaf(v[j].w, v[j].w, fmaf(v[j].z, v[j].z, fmaf(v[j].y, v[j].y, fmaf(v[j].x, v[j].x, acc))));
     acc = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
+    if ((tid & 63) == 0) s_red[tid >> 6] = acc;
     __syncthreads();
     const float ss = ((s_red[0] + s_red[1]) + s_red[2]) + s_red[3];
     const float rms = rsqrtf(ss / (float)n + eps);
-    for (int i = threadIdx.x; i < n; i += 256) o[i] = xr[i] * rms * bf16_to_f32(w[i]);
-}
-
-// ---- GEMM on f32 MFMA -------------------------------------------------------------------
-
-// v_mfma_f32_16x16x4f32: A 16x4 (lane l: row l%16, k l/16), B 4x16 (lane l:
-// column l%16, k l/16), D 16x16 (lane l: column l%16, rows 4(l/16) .. +3).
-// Workgroup tile 64 (tokens) x 64 (weight rows), k-steps of 32; wave w owns
-// the 32 x 32 quarter (w/2, w%2) as 2 x 2 MFMA tiles.  The next k-step's
-// global loads are issued before the current one is computed.
-constexpr int kGM = 64, kGN = 64, kGK = 32;
-
-__global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
-    __shared__ float sA[kGM][kGK + 1];
-    __shared__ float sB[kGN][kGK + 1];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int m0 = blockIdx.y * kGM, n0 = blockIdx.x * kGN;
-    const int lr = tid >> 2, lc = (tid & 3) * 8;  // loader: row, 8 columns
-    const float* arow = g.A + (size_t)min(m0 + lr, g.M - 1) * g.lda + lc;
-    const uint16_t* brow = g.W + (size_t)min(n0 + lr, g.N - 1) * g.K + lc;
-    float4 a0, a1;
-    uint4 b;
-    auto load = [&](int k0) {
-        a0 = *reinterpret_cast<const float4*>(arow + k0);
-        a1 = *reinterpret_cast<const float4*>(arow + k0 + 4);
-        b = *reinterpret_cast<const uint4*>(brow + k0);
-    };
-    f32x4v acc[2][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    const int r16 = lane & 15, k4 = lane >> 4;
-    load(0);
-    for (int k0 = 0; k0 < g.K; k0 += kGK) {
-        sA[lr][lc + 0] = a0.x, sA[lr][lc + 1] = a0.y, sA[lr][lc + 2] = a0.z, sA[lr][lc + 3] = a0.w;
-        sA[lr][lc + 4] = a1.x, sA[lr][lc + 5] = a1.y, sA[lr][lc + 6] = a1.z, sA[lr][lc + 7] = a1.w;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sB[lr][lc + e] = bf16x8_at(b, e);
-        __syncthreads();
-        if (k0 + kGK < g.K) load(k0 + kGK);
-#pragma unroll
-        for (int kk = 0; kk < kGK; kk += 4) {
-            float av[2], bv[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) av[i] = sA[wm + 16 * i + r16][kk + k4];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) bv[j] = sB[wn + 16 * j + r16][kk + k4];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
+    for (int j = 0; j < NV; ++j) {
+        const int i = tid + 256 * j;
+        if (i >= n4) continue;
+        const float y[4] = {v[j].x * rms * bf16_to_f32(b[j].x & 0xFFFFu), v[j].y * rms * bf16_to_f32(b[j].x >> 16),
+                            v[j].z * rms * bf16_to_f32(b[j].y & 0xFFFFu), v[j].w * rms * bf16_to_f32(b[j].y >> 16)};
+        if (parts)
+            store_parts<4>(parts + row + 4 * i, plane, y);
+        else
+            *reinterpret_cast<float4*>(out + row + 4 * i) = float4{y[0], y[1], y[2], y[3]};
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + wn + 16 * j + r16;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = m0 + wm + 16 * i + 4 * k4 + r;
-                if (m < g.M && n < g.N) {
-                    float v = acc[i][j][r];
-                    if (g.R) v += g.R[(size_t)m * g.ldc + n];
-                    g.C[(size_t)m * g.ldc + n] = v;
-                }
-            }
-        }
 }
 
 // ---- q/k norm, RoPE, KV rows ----------------------------------------------------------
@@ -262,9 +244,13 @@ __global__ __launch_bounds__(256) void attn_causal_kernel(PfDenseArgs a) {
         }
     }
     if (live) {
-        float* out = a.attn + (size_t)t * a.qd + (size_t)h * HD;
+        uint16_t* out = a.attn + (size_t)t * a.qd + (size_t)h * HD;
 #pragma unroll
-        for (int e = 0; e < DPT; ++e) out[j + 16 * e] = acc[e] / l;
+        for (int e = 0; e < DPT; ++e) {
+            // (values of the thread's neighbour, so that pairs are stored)
+            const float x = acc[e] / l, y = __shfl_xor(x, 1);
+            if (j % 2 == 0) store_parts<2>(out + j + 16 * e, a.attn_plane, {x, y});
+        }
     }
 }
 
@@ -276,138 +262,143 @@ __global__ void advance_pos_kernel(int32_t* pos, int32_t by, int32_t max_seq) {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16v __attribute__((ext_vector_type(16)));
 
-// Y[M][N] = X[M][K] W[N][K]^T (+ R), X f32, W bf16.  Each x is split exactly
-// into three bf16 values, hi = x with the low 16 bits cleared, mid = (x - hi)
-// likewise, lo = x - hi - mid (x has 24 significant bits: 8 + 8 + 8), when the
-// X tile is staged in LDS; each part is multiplied with the bf16 weights on
-// v_mfma_f32_32x32x16_bf16, whose products are exact, and accumulated in f32:
-// the arithmetic of the f32 GEMM (exact products, f32 sums) at the bf16 rate.
-// Tile BM tokens x BN weight rows (128 x 128, 64 x 128 or 64 x 64), k-blocks
-// of 64; the next k-block's global loads are issued before the current one
-// is multiplied.  Four waves, each TI x TJ tiles of 32 x 32.  MFMA operands:
-// A = tokens (lane l: row l % 32, k 8 (l / 32) .. + 7), B = weight rows
-// likewise; D element 4 v + i of lane l is token 8 v + 4 (l / 32) + i, weight
-// row l % 32 of the tile.
-constexpr int kBK = 64, kBP = kBK + 8;  // LDS rows padded to 144 bytes
-
-template <int BM, int BN>
-__global__ __launch_bounds__(256, 2) void gemm_bf3_kernel(GemmArgs g) {
-    constexpr int TI = BM == 128 ? 2 : (BN == 128 ? 2 : 1);
-    constexpr int TJ = BM == 128 ? 2 : 1;
-    constexpr int WN = BN / (32 * TJ);              // waves along the weight rows
-    static_assert((BM / (32 * TI)) * WN == 4, "four waves");
-    constexpr int EA = BM * kBK / 256;              // X values staged per thread (32 or 16)
-    constexpr int EW = BN * kBK / 256;              // W values staged per thread (32 or 16)
-    __shared__ __attribute__((aligned(16))) uint16_t sX[3][BM][kBP];
-    __shared__ __attribute__((aligned(16))) uint16_t sW[BN][kBP];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    // loaders: X row xr, columns xc .. xc + EA - 1; W row wr, columns wc .. wc + EW - 1
-    const int xr = tid / (kBK / EA), xc = (tid % (kBK / EA)) * EA;
-    const int wr = tid / (kBK / EW), wc = (tid % (kBK / EW)) * EW;
-    const float* xrow = g.A + (size_t)min(m0 + xr, g.M - 1) * g.lda + xc;
-    const int wrow_n = min(n0 + wr, g.N - 1);
-    const uint16_t* wrow = !g.W1 || wrow_n < g.n1 ? g.W + (size_t)wrow_n * g.K + wc
-                           : wrow_n < g.n2        ? g.W1 + (size_t)(wrow_n - g.n1) * g.K + wc
-                                                  : g.W2 + (size_t)(wrow_n - g.n2) * g.K + wc;
-    typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
-    float4 xv[EA / 4];
-    u32x4v wv[EW / 8];
-    // hi / mid / lo parts of eight values, as bf16 bits packed two per word
-    auto split8 = [&](const float (&v)[8], uint4& h, uint4& m, uint4& l) {
-        uint32_t hb[8], mb[8], lb[8];
+// C[M][N] = X[M][K] W[N][K]^T (+ R), X f32 as its three bf16 parts
+// (store_parts), W bf16: each part multiplied with the weights on
+// v_mfma_f32_32x32x16_bf16, whose products are exact, into one f32 accumulator:
+// the arithmetic of the f32 GEMM (exact products, f32 sums) at a third of the
+// bf16 rate.
+// Tile BM tokens x BN weight rows, WM x WN waves of RM x RN blocks of 32 x 32.
+// MFMA A = weight rows, B = tokens (lane l: row l % 32, k 8 (l / 32) .. + 7), so
+// a lane's accumulators are four consecutive outputs of one token.  Every
+// operand byte of a k-block (BK) is copied global -> LDS by the loads
+// themselves (lds_copy16: no registers, no vector work in the loop) into a
+// ring of NS stages, NS - 1 blocks ahead.  A stage is rows of 2 BK bytes, the X
+// parts' then the weights'; 16-byte unit u of row r lies at position u ^ (r & 7)
+// (BK 64) or u ^ ((r >> 2) & 3) (BK 32), so that eight lanes read by one
+// ds_read_b128 hit distinct banks.  Before, f32 tiles were loaded to registers,
+// split and stored to LDS by every workgroup between two barriers per k-block.
+// Bound: MFMA and the operands' way through L2 (a 64 x 128 tile reads 40 KB per
+// 24 MFMAs of each wave).  q, k and v of one layer, N x K 6144 x 2048: T = 37
+// 12.1 -> 12.0 us, 128 19.5 -> 18.8, 333 59.9 -> 45.6, 1000 147 -> 80.5; 6144 x
+// 4096: T = 100 32.6 -> 25.7, 500 139 -> 104, 2048 469 -> 333 (928 TFLOP/s of
+// bf16 products; a plain bf16 product of 8192^3 reaches 1170 here); o_proj, 4096
+// x 4096 at 2048 269 -> 198.
+template <int RM, int RN, int WM, int WN, int BK, int NS>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_parts_kernel(GemmArgs g, int gm, int gn) {
+    constexpr int BM = 32 * RM * WM, BN = 32 * RN * WN, NW = WM * WN;
+    constexpr int RB = 2 * BK, U = BK / 8;                        // bytes and 16-byte units per row
+    constexpr int kX = 3 * BM * RB, kStage = kX + BN * RB;
+    constexpr int kPieces = kStage / 1024, kOps = kPieces / NW;   // 1 KB copies per stage, per wave
+    static_assert(kPieces % NW == 0 && kOps * (NS - 2) < 64, "whole copies per wave");
+    __shared__ __attribute__((aligned(1024))) uint8_t s_ring[NS * kStage];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // an XCD (workgroup id mod 8) takes consecutive tiles, eight token tiles
+    // of each weight tile in a row: their operands meet in its L2
+    const int total = gm * gn, bid = (int)blockIdx.x;
+    const int o = total % 8 == 0 ? (bid & 7) * (total / 8) + (bid >> 3) : bid;
+    const int mg = o / (8 * gn), mh = min(8, gm - 8 * mg), in = o - mg * 8 * gn;
+    const int m0 = (8 * mg + in % mh) * BM, n0 = in / mh * BN;
+    // the weights' segment (its borders are multiples of BN)
+    const uint16_t* w = !g.W1 || n0 < g.n1 ? g.W + (size_t)n0 * g.K
+                        : n0 < g.n2        ? g.W1 + (size_t)(n0 - g.n1) * g.K
+                                           : g.W2 + (size_t)(n0 - g.n2) * g.K;
+    const uint8_t* xb = reinterpret_cast<const uint8_t*>(g.X);
+    const uint8_t* wb = reinterpret_cast<const uint8_t*>(w);
+    auto swizzle = [](int row) { return U == 4 ? (row >> 2) & 3 : row & 7; };
+    uint32_t voff[kOps];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t u = __float_as_uint(v[e]);
-            const float hi = __uint_as_float(u & 0xffff0000u);
-            const float r = v[e] - hi;
-            const float mid = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
-            const float lo = r - mid;
-            hb[e] = __float_as_uint(hi) >> 16;
-            mb[e] = __float_as_uint(mid) >> 16;
-            lb[e] = __float_as_uint(lo) >> 16;
+    for (int i = 0; i < kOps; ++i) {
+        const int row = (64 / U) * (wave * kOps + i) + lane / U;   // of the stage
+        const int u = lane % U ^ swizzle(row);
+        const bool isx = row < 3 * BM;
+        const int r = isx ? row % BM : row - 3 * BM;
+        const uint32_t at = isx ? (uint32_t)min(m0 + r, g.M - 1) : (uint32_t)min(r, g.N - 1 - n0);
+        voff[i] = (isx ? (uint32_t)(row / BM) * (uint32_t)(g.xplane * 2) : 0u) + at * (uint32_t)(g.K * 2) + u * 16;
+    }
+    const int nkb = g.K / BK, S = (int)gridDim.y, z = (int)blockIdx.y;
+    const int kbeg = z * nkb / S, kend = (z + 1) * nkb / S;
+    const uint32_t ring = lds_addr(s_ring);
+    // block kb's copies into its slot (past the last block that block is read
+    // again, into a slot no step reads, so every wave always has the same
+    // number of copies behind a block's)
+    auto issue = [&](int kb, int slot) {
+        const size_t ko = (size_t)min(kb, kend - 1) * RB;
+#pragma unroll
+        for (int i = 0; i < kOps; ++i) {
+            const int p = wave * kOps + i;
+            lds_copy16(voff[i], (p < kX / 1024 ? xb : wb) + ko, ring + slot * kStage + p * 1024);
         }
-        h = make_uint4(hb[0] | hb[1] << 16, hb[2] | hb[3] << 16, hb[4] | hb[5] << 16, hb[6] | hb[7] << 16);
-        m = make_uint4(mb[0] | mb[1] << 16, mb[2] | mb[3] << 16, mb[4] | mb[5] << 16, mb[6] | mb[7] << 16);
-        l = make_uint4(lb[0] | lb[1] << 16, lb[2] | lb[3] << 16, lb[4] | lb[5] << 16, lb[6] | lb[7] << 16);
     };
-    f32x16v acc[TI][TJ];
+    f32x16v acc[RN][RM];
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+    for (int j = 0; j < RN; ++j)
 #pragma unroll
-        for (int j = 0; j < TJ; ++j)
+        for (int i = 0; i < RM; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    const int wm = (wave / WN) * 32 * TI, wn = (wave % WN) * 32 * TJ;
-    const int r32 = lane & 31, k8 = (lane >> 5) * 8;
-    // this workgroup's k range: split blockIdx.z of gridDim.z, whole k-blocks
-    const int nkb = g.K / kBK, S = (int)gridDim.z, z = (int)blockIdx.z;
-    const int kbeg = (z * nkb / S) * kBK, kend = ((z + 1) * nkb / S) * kBK;
+            for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
+    const int r32 = lane & 31, h = lane >> 5, wm = (wave % WM) * 32 * RM, wn = (wave / WM) * 32 * RN;
+    const int sw = swizzle(r32);
 #pragma unroll
-    for (int i = 0; i < EA / 4; ++i) xv[i] = *reinterpret_cast<const float4*>(xrow + kbeg + 4 * i);
+    for (int s = 0; s < NS - 1; ++s) issue(kbeg + s, s);
+    int slot = 0;
+    for (int kb = kbeg; kb < kend; ++kb) {
+        wait_vm<kOps * (NS - 2)>();   // block kb's copies are in (the next NS - 2 may not be)
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        issue(kb + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t* st = s_ring + slot * kStage;
+        // the operands of k-step ks + 1 are read while step ks is multiplied
+        bf16x8 af[2][RN], bf[2][3][RM];
+        auto read = [&](int ks, int at) {
+            const int u = ((2 * ks + h) ^ sw) * 16;
 #pragma unroll
-    for (int i = 0; i < EW / 8; ++i) wv[i] = *reinterpret_cast<const u32x4v*>(wrow + kbeg + 8 * i);
-    for (int k0 = kbeg; k0 < kend; k0 += kBK) {
-#pragma unroll
-        for (int c = 0; c < EA / 8; ++c) {
-            float v[8];
-            v[0] = xv[2 * c].x, v[1] = xv[2 * c].y, v[2] = xv[2 * c].z, v[3] = xv[2 * c].w;
-            v[4] = xv[2 * c + 1].x, v[5] = xv[2 * c + 1].y, v[6] = xv[2 * c + 1].z, v[7] = xv[2 * c + 1].w;
-            uint4 h, m, l;
-            split8(v, h, m, l);
-            *reinterpret_cast<uint4*>(&sX[0][xr][xc + 8 * c]) = h;
-            *reinterpret_cast<uint4*>(&sX[1][xr][xc + 8 * c]) = m;
-            *reinterpret_cast<uint4*>(&sX[2][xr][xc + 8 * c]) = l;
-        }
-#pragma unroll
-        for (int c = 0; c < EW / 8; ++c) *reinterpret_cast<u32x4v*>(&sW[wr][wc + 8 * c]) = wv[c];
-        __syncthreads();
-        if (k0 + kBK < kend) {
-            const int k1 = k0 + kBK;
-#pragma unroll
-            for (int i = 0; i < EA / 4; ++i) xv[i] = *reinterpret_cast<const float4*>(xrow + k1 + 4 * i);
-#pragma unroll
-            for (int i = 0; i < EW / 8; ++i) wv[i] = *reinterpret_cast<const u32x4v*>(wrow + k1 + 8 * i);
-        }
-#pragma unroll
-        for (int ks = 0; ks < kBK; ks += 16) {
-            bf16x8 b[TJ];
-#pragma unroll
-            for (int j = 0; j < TJ; ++j)
-                b[j] = *reinterpret_cast<const bf16x8*>(&sW[wn + 32 * j + r32][ks + k8]);
+            for (int j = 0; j < RN; ++j)
+                af[at][j] = *reinterpret_cast<const bf16x8*>(st + kX + (wn + 32 * j + r32) * RB + u);
 #pragma unroll
             for (int p = 0; p < 3; ++p)
 #pragma unroll
-                for (int i = 0; i < TI; ++i) {
-                    const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sX[p][wm + 32 * i + r32][ks + k8]);
+                for (int i = 0; i < RM; ++i)
+                    bf[at][p][i] = *reinterpret_cast<const bf16x8*>(st + (p * BM + wm + 32 * i + r32) * RB + u);
+        };
+        read(0, 0);
 #pragma unroll
-                    for (int j = 0; j < TJ; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[j], acc[i][j], 0, 0, 0);
-                }
+        for (int ks = 0; ks < BK / 16; ++ks) {
+            if (ks + 1 < BK / 16) read(ks + 1, (ks + 1) & 1);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int i = 0; i < RM; ++i)
+#pragma unroll
+                    for (int j = 0; j < RN; ++j)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][j], bf[ks & 1][p][i],
+                                                                            acc[j][i], 0, 0, 0);
         }
-        __syncthreads();
+        slot = slot + 1 == NS ? 0 : slot + 1;
     }
+    wait_vm<0>();   // no copy into LDS may still be in flight when the workgroup ends
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+    for (int i = 0; i < RM; ++i) {
+        const int m = m0 + wm + 32 * i + r32;
+        if (m >= g.M) continue;
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const int n = n0 + wn + 32 * j + r32;
+        for (int j = 0; j < RN; ++j)
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = m0 + wm + 32 * i + 8 * v + 4 * (lane >> 5) + r;
-                    if (m < g.M && n < g.N) {
-                        float y = acc[i][j][4 * v + r];
-                        if (S > 1) {
-                            g.part[((size_t)z * g.M + m) * g.N + n] = y;
-                        } else {
-                            if (g.R) y += g.R[(size_t)m * g.ldc + n];
-                            g.C[(size_t)m * g.ldc + n] = y;
-                        }
+            for (int v = 0; v < 4; ++v) {
+                const int n = n0 + wn + 32 * j + 8 * v + 4 * h;
+                if (n >= g.N) continue;   // (N % 4 == 0)
+                float4 y{acc[j][i][4 * v], acc[j][i][4 * v + 1], acc[j][i][4 * v + 2], acc[j][i][4 * v + 3]};
+                if (S > 1) {
+                    *reinterpret_cast<float4*>(g.part + ((size_t)z * g.M + m) * g.N + n) = y;
+                } else {
+                    if (g.R) {
+                        const float4 r = *reinterpret_cast<const float4*>(g.R + (size_t)m * g.ldc + n);
+                        y.x += r.x, y.y += r.y, y.z += r.z, y.w += r.w;
                     }
+                    *reinterpret_cast<float4*>(g.C + (size_t)m * g.ldc + n) = y;
                 }
-        }
+            }
+    }
 }
 
 // C = sum over s = 0 .. S-1 of the split-K partials (in that order) + R; four
@@ -468,6 +459,8 @@ __global__ __launch_bounds__(256) void splitk_sum_norm_kernel(GemmArgs g) {
     for (int i = threadIdx.x; i < g.N; i += 256) o[i] = c[i] * rms * bf16_to_f32(g.norm_w[i]);
 }
 
+constexpr long kGemmSplitWgs = 512;   // workgroups of a split grid
+
 }  // namespace
 
 int launch_pf_embed(const PfDenseArgs& a, void* stream) {
@@ -475,59 +468,76 @@ int launch_pf_embed(const PfDenseArgs& a, void* stream) {
     return (int)hipGetLastError();
 }
 
-int launch_rmsnorm_rows(const float* x, const uint16_t* w, float* out, int rows, int n, float eps,
-                        void* stream) {
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)rows), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       x, w, out, n, eps);
+int launch_rmsnorm_rows(const float* x, const uint16_t* w, float* out, uint16_t* parts, int64_t plane, int rows,
+                        int n, float eps, void* stream) {
+    if (n % 4 || n <= 0 || n > 8192) return (int)hipErrorInvalidValue;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const dim3 grid((unsigned)rows);
+    if (n <= 2048)
+        hipLaunchKernelGGL(rmsnorm_rows_kernel<2>, grid, dim3(256), 0, st, x, w, out, parts, plane, n, eps);
+    else if (n <= 4096)
+        hipLaunchKernelGGL(rmsnorm_rows_kernel<4>, grid, dim3(256), 0, st, x, w, out, parts, plane, n, eps);
+    else
+        hipLaunchKernelGGL(rmsnorm_rows_kernel<8>, grid, dim3(256), 0, st, x, w, out, parts, plane, n, eps);
     return (int)hipGetLastError();
 }
 
-int launch_gemm(const GemmArgs& g, void* stream) {
-    if (g.K % kGK || g.M <= 0 || g.N <= 0 || g.lda % 4) return (int)hipErrorInvalidValue;
-    if (g.W1 && (g.K % kBK || !g.W2 || g.n1 < 0 || g.n1 > g.n2 || g.n2 > g.N))
+namespace {
+template <int RM, int RN, int WM, int WN, int BK, int NS>
+void launch_gemm_tile(const GemmArgs& g, hipStream_t st) {
+    const int gm = (g.M + 32 * RM * WM - 1) / (32 * RM * WM), gn = (g.N + 32 * RN * WN - 1) / (32 * RN * WN);
+    hipLaunchKernelGGL((gemm_parts_kernel<RM, RN, WM, WN, BK, NS>), dim3((unsigned)(gm * gn), (unsigned)g.splits),
+                       dim3(64 * WM * WN), 0, st, g, gm, gn);
+}
+}  // namespace
+
+int launch_gemm(const GemmArgs& g0, void* stream) {
+    GemmArgs g = g0;
+    if (g.K % 64 || g.K <= 0 || g.M <= 0 || g.N <= 0 || g.N % 4 || g.ldc % 4 || (uintptr_t)g.C % 16 ||
+        (uintptr_t)g.R % 16 || g.xplane < (int64_t)g.M * g.K || 6 * g.xplane >= (1ll << 32) ||
+        2ll * 128 * g.K >= (1ll << 32))
+        return (int)hipErrorInvalidValue;
+    if (g.W1 && (!g.W2 || g.n1 < 0 || g.n1 > g.n2 || g.n2 > g.N || g.n1 % 64 || g.n2 % 64))
         return (int)hipErrorInvalidValue;
     if (g.norm_w && (!g.norm_out || g.ldc != g.N)) return (int)hipErrorInvalidValue;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    int splits = 1;
-    if (g.K % kBK) {  // f32 MFMA for a K that is not a multiple of 64
-        const dim3 grid((unsigned)((g.N + kGN - 1) / kGN), (unsigned)((g.M + kGM - 1) / kGM));
-        hipLaunchKernelGGL(gemm_kernel, grid, dim3(256), 0, st, g);
+    // Tiles of 64 x 128, two workgroups per CU: measured best or within a few
+    // percent at every size but one, a grid of 128 x 256 tiles that is nearly
+    // one full round of the CUs (2048 x 4096 x 4096: 256 of them 200 us, 1024 of
+    // 64 x 128 215; 1100 x 6144 x 4096, 216: 175 against 207; but 192 of them at
+    // 1000 x 6144 x 2048 84 against 82, 384 at 2048 x 6144 x 4096 342 against
+    // 307).  The weight segments' borders must be tile borders.
+    const bool wide = !g.W1 || (g.n1 % 128 == 0 && g.n2 % 128 == 0);
+    const bool wide256 = !g.W1 || (g.n1 % 256 == 0 && g.n2 % 256 == 0);
+    const long gm64 = (g.M + 63) / 64, gn128 = (g.N + 127) / 128, gn64 = (g.N + 63) / 64;
+    const long big = (long)((g.M + 127) / 128) * ((g.N + 255) / 256);
+    g.splits = 1;
+    if (wide256 && big > 208 && big <= 256) {
+        launch_gemm_tile<2, 2, 2, 4, 32, 3>(g, st);
     } else {
-        // the largest tile that still gives at least one workgroup per CU
-        const long gm128 = (g.M + 127) / 128, gm64 = (g.M + 63) / 64;
-        const long gn128 = (g.N + 127) / 128, gn64 = (g.N + 63) / 64;
-        if (gn128 * gm128 >= 256) {
-            hipLaunchKernelGGL((gemm_bf3_kernel<128, 128>), dim3((unsigned)gn128, (unsigned)gm128),
-                               dim3(256), 0, st, g);
-        } else if (gn128 * gm64 >= 256) {
-            hipLaunchKernelGGL((gemm_bf3_kernel<64, 128>), dim3((unsigned)gn128, (unsigned)gm64),
-                               dim3(256), 0, st, g);
-        } else {
-            // Too few 64 x 64 tiles to fill the chip: split the k-blocks over
-            // gridDim.z (at least 4 per split, at most 512 workgroups in all)
-            // and sum the partials in a fixed order, so results do not depend
-            // on timing.
-            const long tiles = gn64 * gm64, nkb = g.K / kBK;
-            long S = 768 / tiles < nkb / 4 ? 768 / tiles : nkb / 4;
-            const bool aligned = g.N % 4 == 0 && g.ldc % 4 == 0 && (uintptr_t)g.C % 16 == 0 &&
-                                 (uintptr_t)g.R % 16 == 0;
-            if (!g.part || !aligned || S < 2 || S * g.M * g.N > kGemmPartFloats) S = 1;
-            GemmArgs gs = g;
-            gs.splits = splits = (int)S;
-            hipLaunchKernelGGL((gemm_bf3_kernel<64, 64>),
-                               dim3((unsigned)gn64, (unsigned)gm64, (unsigned)S), dim3(256), 0, st, gs);
-            if (S > 1 && S <= kSumNormSplits && g.norm_w) {  // the sum makes the row norm too
-                hipLaunchKernelGGL(splitk_sum_norm_kernel, dim3((unsigned)g.M), dim3(256), 0, st, gs);
-            } else if (S > 1) {
-                const size_t mn4 = (size_t)g.M * g.N / 4;
-                hipLaunchKernelGGL(splitk_sum_kernel, dim3((unsigned)((mn4 + 255) / 256)), dim3(256), 0,
-                                   st, gs);
-            }
+        // Tiles of 64 tokens; too few of them: the k-blocks are split over
+        // gridDim.y (at least 4 blocks of 64 per split, at most
+        // kGemmSplitWgs workgroups in all) and the partials summed in a fixed
+        // order, so results do not depend on timing.
+        const long tiles = wide ? gn128 * gm64 : gn64 * gm64, nkb = g.K / 64;
+        long S = tiles < 256 ? std::min(kGemmSplitWgs / tiles, nkb / 4) : 1;
+        if (g.part) S = std::min(S, (long)(kGemmPartFloats / ((int64_t)g.M * g.N)));
+        if (!g.part || S < 2) S = 1;
+        g.splits = (int)S;
+        if (wide)
+            launch_gemm_tile<1, 2, 2, 2, 64, 2>(g, st);
+        else
+            launch_gemm_tile<1, 1, 2, 2, 64, 2>(g, st);
+        if (S > 1 && S <= kSumNormSplits && g.norm_w) {  // the sum makes the row norm too
+            hipLaunchKernelGGL(splitk_sum_norm_kernel, dim3((unsigned)g.M), dim3(256), 0, st, g);
+        } else if (S > 1) {
+            const size_t mn4 = (size_t)g.M * g.N / 4;
+            hipLaunchKernelGGL(splitk_sum_kernel, dim3((unsigned)((mn4 + 255) / 256)), dim3(256), 0, st, g);
         }
     }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !g.norm_w || (splits > 1 && splits <= kSumNormSplits)) return (int)e;
-    return launch_rmsnorm_rows(g.C, g.norm_w, g.norm_out, g.M, g.N, g.norm_eps, stream);
+    if (e != hipSuccess || !g.norm_w || (g.splits > 1 && g.splits <= kSumNormSplits)) return (int)e;
+    return launch_rmsnorm_rows(g.C, g.norm_w, g.norm_out, nullptr, 0, g.M, g.N, g.norm_eps, stream);
 }
 
 int launch_pf_rope_kv(const PfDenseArgs& a, void* stream) {
@@ -844,10 +854,10 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(PfDenseArgs a) {
     }
     if (t0 + w.r32 >= a.T) return;
     // wave w: accumulator rows 8 w + 4 h .. + 3 of every tile
-    float* out = a.attn + (size_t)w.t * a.qd + (size_t)head * HD;
+    uint16_t* out = a.attn + (size_t)w.t * a.qd + (size_t)head * HD;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        vecT o;
+        float o[NT];
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
             float x = 0.f;
@@ -856,7 +866,7 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(PfDenseArgs a) {
                 x = fmaf(sO[(k * 16 * NT + (4 * wave + v) * NT + i) * 64 + lane], f[k], x);
             o[i] = x / L;
         }
-        *reinterpret_cast<vecT*>(out + NT * (8 * wave + 4 * w.h + v)) = o;
+        store_parts<NT>(out + NT * (8 * wave + 4 * w.h + v), a.attn_plane, o);
     }
 }
 
