@@ -594,6 +594,7 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
     a.embed = dec->embed;
     a.res = dec->pf_res;
     a.qkv = dec->pf_qkv;
+    a.rope = dec->rope;
     a.attn = dec->pf_parts;
     a.attn_plane = (int64_t)T * qd;
     a.pos = dec->pos;
@@ -628,6 +629,9 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
         g.N = N;
         g.K = h;
         g.part = dec->pf_part;
+        // (split partials are summed by launch_pf_rope_kv)
+        a.part = dec->pf_part;
+        a.splits = gemm_splits(g);
         return launched(launch_gemm(g, st), "prefill q/k/v");
     };
     if ((rc = launched(launch_pf_embed(a, st), "prefill embedding"))) return rc;  // :129-131

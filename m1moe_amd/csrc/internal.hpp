@@ -391,8 +391,10 @@ struct GemmArgs {
     float* C;
     int32_t ldc;
     int32_t M, N, K;
-    // split-K workspace ([S][M][N] f32 partials, summed in order s = 0 .. S-1)
-    // or null; with it a GEMM whose tiles leave the CUs idle splits its k range
+    // split-K workspace ([S][M][N] f32 partials, to be summed in the order s =
+    // 0 .. S-1) or null; with it a GEMM whose tiles leave the CUs idle splits
+    // its k range (gemm_splits).  With norm_w launch_gemm sums them into C,
+    // without it they are left for the caller's next launch
     float* part;
     int32_t splits;              // set by launch_gemm
     // optional second and third weight segments: rows [n1, n2) are rows
@@ -408,6 +410,7 @@ struct GemmArgs {
     float* norm_out;
     float norm_eps;
 };
+constexpr int kGemmMaxSplits = 8;
 constexpr int64_t kGemmPartFloats = 768LL * 64 * 64;  // the workspace launch_gemm may use
 
 // The T prompt tokens of a decoder prefill at positions *pos .. *pos + T - 1.
@@ -416,6 +419,9 @@ struct PfDenseArgs {
     const uint16_t* embed;       // [vocab][h]
     float* res;                  // [T][h] residual stream
     float* qkv;                  // [T][ldqkv]: q | k | v
+    const float* part;           // splits > 1: the projections as the GEMM's partials [splits][T][ldqkv]
+    int32_t splits;
+    const float* rope;           // [max_seq][head_dim / 2] (cos, sin)
     uint16_t* attn;              // output: three bf16 parts (GemmArgs::X), each [T][qd]
     int64_t attn_plane;          // values between the parts
     const uint16_t* q_norm;      // [head_dim] or null
@@ -435,6 +441,8 @@ int launch_pf_embed(const PfDenseArgs& a, void* stream);
 int launch_rmsnorm_rows(const float* x, const uint16_t* w, float* out, uint16_t* parts, int64_t plane, int rows,
                         int n, float eps, void* stream);
 int launch_gemm(const GemmArgs& g, void* stream);
+// The k splits launch_gemm makes of g (1: C is written by the GEMM itself).
+int gemm_splits(const GemmArgs& g);
 int launch_pf_rope_kv(const PfDenseArgs& a, void* stream);
 int launch_pf_attention(const PfDenseArgs& a, void* stream);
 int launch_advance_pos(int32_t* pos, int32_t by, int32_t max_seq, void* stream);

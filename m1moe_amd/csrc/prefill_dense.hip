@@ -120,50 +120,86 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* x, const
 
 // ---- q/k norm, RoPE, KV rows ----------------------------------------------------------
 
-// Workgroup (t, head): head < num_heads: q head, rotated in place; else kv
-// head: k normalised and rotated, k and v stored at cache row p0 + t.
+// Token blockIdx.x, heads kRopeHeads blockIdx.y .. (the q heads, then the kv
+// heads): a q head rotated into qkv, a kv head's k normalised and rotated, k
+// and v stored at cache row p0 + t.  G lanes per head, lane i with dims i, i +
+// G, .. and their partners HD / 2 on: whole 64-lane rows of loads, no LDS.  The
+// projections come as qkv, or as the GEMM's split partials (splits > 1), summed
+// here in the order s = 0 .. S - 1; cos and sin from the decoder's table
+// (rope_table_kernel).  Bound by the bytes at long prompts (32 + 8 heads of
+// 128, T = 2048: 30.9 -> 19.4 us for 100 MB; before, one wave per head computed
+// the powers, sines and cosines of its angles); 16 + 16 heads T = 333 8.8 -> 6.8,
+// T = 128 with 4 splits 5.0 + 5.0 for their own sum -> 7.5.
+constexpr int kRopeHeads = 8;
 template <int HD>
-__global__ __launch_bounds__(64) void rope_kv_rows_kernel(PfDenseArgs a) {
-    __shared__ float s_v[HD];
-    const int t = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
-    const int p = *a.pos + t;
-    const bool is_q = head < a.num_heads;
-    const int kvh = head - a.num_heads;
-    float* row = a.qkv + (size_t)t * a.ldqkv;
-    float* vec = is_q ? row + (size_t)head * HD : row + a.qd + (size_t)kvh * HD;
-    const uint16_t* nw = is_q ? a.q_norm : a.k_norm;
+__global__ __launch_bounds__(256) void rope_kv_rows_kernel(PfDenseArgs a) {
+    constexpr int H2 = HD / 2, G = H2 < 64 ? H2 : 64, NP = H2 / G;   // lanes per head, pairs per lane
+    constexpr int kSlots = 256 / G, PASS = (kRopeHeads + kSlots - 1) / kSlots;
+    const int t = blockIdx.x, slot = threadIdx.x / G, i = threadIdx.x % G;
+    const int p = *a.pos + t, heads = a.num_heads + a.num_kv_heads;
     if (p >= a.max_seq) {
-        if (lane == 0 && head == 0) flag_error(a.err, 32u);
+        if (threadIdx.x == 0 && blockIdx.y == 0) flag_error(a.err, 32u);
         return;
     }
-    float v[HD / 64];
-    float ss = 0.f;
+    // value at column c of the token's projections
+    const size_t at = (size_t)t * a.ldqkv, step = (size_t)a.T * a.ldqkv;
+    auto value = [&](int c) {
+        if (a.splits <= 1) return a.qkv[at + c];
+        float y[kGemmMaxSplits];   // every split's load in flight together
 #pragma unroll
-    for (int j = 0; j < HD / 64; ++j) {
-        v[j] = vec[lane + 64 * j];
-        ss = fmaf(v[j], v[j], ss);
-    }
-    if (nw) {
-        const float rms = 1.0f / sqrtf(wave_sum(ss) / (float)HD + a.eps);
+        for (int z = 0; z < kGemmMaxSplits; ++z)
+            if (z < a.splits) y[z] = a.part[z * step + at + c];
+        float v = y[0];
 #pragma unroll
-        for (int j = 0; j < HD / 64; ++j) v[j] *= rms * bf16_to_f32(nw[lane + 64 * j]);
-    }
+        for (int z = 1; z < kGemmMaxSplits; ++z)
+            if (z < a.splits) v += y[z];
+        return v;
+    };
 #pragma unroll
-    for (int j = 0; j < HD / 64; ++j) s_v[lane + 64 * j] = v[j];
-    __syncthreads();
-    float* dst = is_q ? vec : a.kcache + (size_t)p * a.kvd + (size_t)kvh * HD;
-    for (int d = lane; d < HD / 2; d += 64) {
-        const float freq = 1.0f / powf(a.rope_theta, (float)(2 * d) / (float)HD);
-        const float ang = (float)p * freq;
-        const float cs = cosf(ang), sn = sinf(ang);
-        const float x0 = s_v[d], x1 = s_v[d + HD / 2];
-        dst[d] = x0 * cs - x1 * sn;
-        dst[d + HD / 2] = x0 * sn + x1 * cs;
-    }
-    if (!is_q) {
-        const float* vsrc = row + a.qd + a.kvd + (size_t)kvh * HD;
+    for (int k = 0; k < PASS; ++k) {
+        const int head = kRopeHeads * (int)blockIdx.y + k * kSlots + slot;
+        if (head >= heads) continue;   // (uniform over the head's lanes)
+        const bool is_q = head < a.num_heads;
+        const int kvh = head - a.num_heads;
+        const int c0 = is_q ? head * HD : a.qd + kvh * HD;
+        const uint16_t* nw = is_q ? a.q_norm : a.k_norm;
+        float x0[NP], x1[NP], v0[NP], v1[NP];
+        float2 r[NP];
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int d = i + G * j;
+            x0[j] = value(c0 + d);
+            x1[j] = value(c0 + d + H2);
+            if (!is_q) {
+                v0[j] = value(c0 + a.kvd + d);
+                v1[j] = value(c0 + a.kvd + d + H2);
+            }
+            r[j] = reinterpret_cast<const float2*>(a.rope)[(size_t)p * H2 + d];
+            ss = fmaf(x0[j], x0[j], fmaf(x1[j], x1[j], ss));
+        }
+        if (nw) {
+#pragma unroll
+            for (int o = 1; o < G; o <<= 1) ss += __shfl_xor(ss, o);
+            const float rms = 1.0f / sqrtf(ss / (float)HD + a.eps);
+#pragma unroll
+            for (int j = 0; j < NP; ++j) {
+                x0[j] *= rms * bf16_to_f32(nw[i + G * j]);
+                x1[j] *= rms * bf16_to_f32(nw[i + G * j + H2]);
+            }
+        }
+        float* dst = is_q ? a.qkv + at + c0 : a.kcache + (size_t)p * a.kvd + (size_t)kvh * HD;
         float* vdst = a.vcache + (size_t)p * a.kvd + (size_t)kvh * HD;
-        for (int d = lane; d < HD; d += 64) vdst[d] = vsrc[d];
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int d = i + G * j;
+            dst[d] = x0[j] * r[j].x - x1[j] * r[j].y;
+            dst[d + H2] = x0[j] * r[j].y + x1[j] * r[j].x;
+            if (!is_q) {
+                vdst[d] = v0[j];
+                vdst[d + H2] = v1[j];
+            }
+        }
     }
 }
 
@@ -401,30 +437,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_parts_kernel(GemmArgs g,
     }
 }
 
-// C = sum over s = 0 .. S-1 of the split-K partials (in that order) + R; four
-// columns per thread (N, ldc and the C / R addresses are multiples of 4).
-__global__ __launch_bounds__(256) void splitk_sum_kernel(GemmArgs g) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t mn4 = (size_t)g.M * g.N / 4;
-    if (i >= mn4) return;
-    const float4* p = reinterpret_cast<const float4*>(g.part);
-    float4 y = p[i];
-    for (int z = 1; z < g.splits; ++z) {
-        const float4 q = p[(size_t)z * mn4 + i];
-        y.x += q.x, y.y += q.y, y.z += q.z, y.w += q.w;
-    }
-    const size_t m = 4 * i / g.N, n = 4 * i % g.N;
-    if (g.R) {
-        const float4 r = *reinterpret_cast<const float4*>(g.R + m * g.ldc + n);
-        y.x += r.x, y.y += r.y, y.z += r.z, y.w += r.w;
-    }
-    *reinterpret_cast<float4*>(g.C + m * g.ldc + n) = y;
-}
-
-// The same sum for one output row per workgroup (at most kSumNormSplits
-// splits), then that row's RMSNorm with the arithmetic of rmsnorm_rows_kernel
+// C = sum over s = 0 .. S-1 of the split-K partials (in that order, at most
+// kGemmMaxSplits) + R, one output row per workgroup, then that row's RMSNorm with the arithmetic of rmsnorm_rows_kernel
 // (each thread's squares summed in its own column order, four at a time).
-constexpr int kSumNormSplits = 8;
 __global__ __launch_bounds__(256) void splitk_sum_norm_kernel(GemmArgs g) {
     __shared__ float s_red[4];
     const size_t m = blockIdx.x, mn4 = (size_t)g.M * g.N / 4;
@@ -432,13 +447,13 @@ __global__ __launch_bounds__(256) void splitk_sum_norm_kernel(GemmArgs g) {
     float* c = g.C + m * g.ldc;
     float acc = 0.f;
     for (int i = threadIdx.x; i < g.N / 4; i += 256) {
-        float4 v[kSumNormSplits];  // every split's load in flight together
+        float4 v[kGemmMaxSplits];  // every split's load in flight together
 #pragma unroll
-        for (int z = 0; z < kSumNormSplits; ++z)
+        for (int z = 0; z < kGemmMaxSplits; ++z)
             if (z < g.splits) v[z] = p[(size_t)z * mn4 + i];
         float4 y = v[0];
 #pragma unroll
-        for (int z = 1; z < kSumNormSplits; ++z)
+        for (int z = 1; z < kGemmMaxSplits; ++z)
             if (z < g.splits) y.x += v[z].x, y.y += v[z].y, y.z += v[z].z, y.w += v[z].w;
         if (g.R) {
             const float4 r = *reinterpret_cast<const float4*>(g.R + m * g.ldc + 4 * i);
@@ -491,6 +506,36 @@ void launch_gemm_tile(const GemmArgs& g, hipStream_t st) {
 }
 }  // namespace
 
+namespace {
+// Tiles of 64 x 128, two workgroups per CU: measured best or within a few
+// percent at every size but one, a grid of 128 x 256 tiles that is nearly one
+// full round of the CUs (2048 x 4096 x 4096: 256 of them 200 us, 1024 of 64 x
+// 128 215; 1100 x 6144 x 4096, 216: 175 against 207; but 192 of them at 1000 x
+// 6144 x 2048 84 against 82, 384 at 2048 x 6144 x 4096 342 against 307).  The
+// weight segments' borders must be tile borders.  Too few tiles: the k-blocks
+// are split over gridDim.y (at least 4 blocks of 64 per split, at most
+// kGemmSplitWgs workgroups in all) and the partials summed in a fixed order,
+// so results do not depend on timing.
+struct GemmPlan {
+    bool big, wide;
+    int splits;
+};
+GemmPlan gemm_plan(const GemmArgs& g) {
+    const long gm64 = (g.M + 63) / 64, gn128 = (g.N + 127) / 128, gn64 = (g.N + 63) / 64;
+    const long big = (long)((g.M + 127) / 128) * ((g.N + 255) / 256);
+    GemmPlan p{};
+    p.wide = !g.W1 || (g.n1 % 128 == 0 && g.n2 % 128 == 0);
+    p.big = big > 208 && big <= 256 && (!g.W1 || (g.n1 % 256 == 0 && g.n2 % 256 == 0));
+    const long tiles = p.wide ? gn128 * gm64 : gn64 * gm64, nkb = g.K / 64;
+    long S = !p.big && g.part && tiles < 256 ? std::min(kGemmSplitWgs / tiles, nkb / 4) : 1;
+    S = std::min({S, (long)kGemmMaxSplits, (long)(kGemmPartFloats / ((int64_t)g.M * g.N))});
+    p.splits = (int)std::max(S, 1l);
+    return p;
+}
+}  // namespace
+
+int gemm_splits(const GemmArgs& g) { return gemm_plan(g).splits; }
+
 int launch_gemm(const GemmArgs& g0, void* stream) {
     GemmArgs g = g0;
     if (g.K % 64 || g.K <= 0 || g.M <= 0 || g.N <= 0 || g.N % 4 || g.ldc % 4 || (uintptr_t)g.C % 16 ||
@@ -501,52 +546,29 @@ int launch_gemm(const GemmArgs& g0, void* stream) {
         return (int)hipErrorInvalidValue;
     if (g.norm_w && (!g.norm_out || g.ldc != g.N)) return (int)hipErrorInvalidValue;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Tiles of 64 x 128, two workgroups per CU: measured best or within a few
-    // percent at every size but one, a grid of 128 x 256 tiles that is nearly
-    // one full round of the CUs (2048 x 4096 x 4096: 256 of them 200 us, 1024 of
-    // 64 x 128 215; 1100 x 6144 x 4096, 216: 175 against 207; but 192 of them at
-    // 1000 x 6144 x 2048 84 against 82, 384 at 2048 x 6144 x 4096 342 against
-    // 307).  The weight segments' borders must be tile borders.
-    const bool wide = !g.W1 || (g.n1 % 128 == 0 && g.n2 % 128 == 0);
-    const bool wide256 = !g.W1 || (g.n1 % 256 == 0 && g.n2 % 256 == 0);
-    const long gm64 = (g.M + 63) / 64, gn128 = (g.N + 127) / 128, gn64 = (g.N + 63) / 64;
-    const long big = (long)((g.M + 127) / 128) * ((g.N + 255) / 256);
-    g.splits = 1;
-    if (wide256 && big > 208 && big <= 256) {
+    const GemmPlan plan = gemm_plan(g);
+    g.splits = plan.splits;
+    if (plan.big)
         launch_gemm_tile<2, 2, 2, 4, 32, 3>(g, st);
-    } else {
-        // Tiles of 64 tokens; too few of them: the k-blocks are split over
-        // gridDim.y (at least 4 blocks of 64 per split, at most
-        // kGemmSplitWgs workgroups in all) and the partials summed in a fixed
-        // order, so results do not depend on timing.
-        const long tiles = wide ? gn128 * gm64 : gn64 * gm64, nkb = g.K / 64;
-        long S = tiles < 256 ? std::min(kGemmSplitWgs / tiles, nkb / 4) : 1;
-        if (g.part) S = std::min(S, (long)(kGemmPartFloats / ((int64_t)g.M * g.N)));
-        if (!g.part || S < 2) S = 1;
-        g.splits = (int)S;
-        if (wide)
-            launch_gemm_tile<1, 2, 2, 2, 64, 2>(g, st);
-        else
-            launch_gemm_tile<1, 1, 2, 2, 64, 2>(g, st);
-        if (S > 1 && S <= kSumNormSplits && g.norm_w) {  // the sum makes the row norm too
-            hipLaunchKernelGGL(splitk_sum_norm_kernel, dim3((unsigned)g.M), dim3(256), 0, st, g);
-        } else if (S > 1) {
-            const size_t mn4 = (size_t)g.M * g.N / 4;
-            hipLaunchKernelGGL(splitk_sum_kernel, dim3((unsigned)((mn4 + 255) / 256)), dim3(256), 0, st, g);
-        }
-    }
+    else if (plan.wide)
+        launch_gemm_tile<1, 2, 2, 2, 64, 2>(g, st);
+    else
+        launch_gemm_tile<1, 1, 2, 2, 64, 2>(g, st);
+    if (g.splits > 1 && g.norm_w)  // the sum makes the row norm too
+        hipLaunchKernelGGL(splitk_sum_norm_kernel, dim3((unsigned)g.M), dim3(256), 0, st, g);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !g.norm_w || (g.splits > 1 && g.splits <= kSumNormSplits)) return (int)e;
+    if (e != hipSuccess || !g.norm_w || g.splits > 1) return (int)e;
     return launch_rmsnorm_rows(g.C, g.norm_w, g.norm_out, nullptr, 0, g.M, g.N, g.norm_eps, stream);
 }
 
 int launch_pf_rope_kv(const PfDenseArgs& a, void* stream) {
-    const dim3 grid((unsigned)a.T, (unsigned)(a.num_heads + a.num_kv_heads));
+    if (!a.rope || (a.splits > 1 && (!a.part || a.splits > kGemmMaxSplits))) return (int)hipErrorInvalidValue;
+    const dim3 grid((unsigned)a.T, (unsigned)((a.num_heads + a.num_kv_heads + kRopeHeads - 1) / kRopeHeads));
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (a.head_dim) {
-        case 64: hipLaunchKernelGGL(rope_kv_rows_kernel<64>, grid, dim3(64), 0, st, a); break;
-        case 128: hipLaunchKernelGGL(rope_kv_rows_kernel<128>, grid, dim3(64), 0, st, a); break;
-        case 256: hipLaunchKernelGGL(rope_kv_rows_kernel<256>, grid, dim3(64), 0, st, a); break;
+        case 64: hipLaunchKernelGGL(rope_kv_rows_kernel<64>, grid, dim3(256), 0, st, a); break;
+        case 128: hipLaunchKernelGGL(rope_kv_rows_kernel<128>, grid, dim3(256), 0, st, a); break;
+        case 256: hipLaunchKernelGGL(rope_kv_rows_kernel<256>, grid, dim3(256), 0, st, a); break;
         default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();
