@@ -5,11 +5,12 @@
 // sync.  Two kernels:
 //
 //   router_logits   logits[t][e] = sum_d W[e][d] * x[t][d]: a wave computes
-//                   4 tokens x 4 experts with its lanes across the columns
-//                   (coalesced 128-bit loads, all of a 2048-column row in
-//                   flight at once), a workgroup 4 tokens x 16 experts.  For
-//                   a prefill an extra row of workgroups writes x's f16 copy
-//                   (prep_token): wave w takes token t0 + w.
+//                   TT tokens x 4 experts (TT 4, or 2 or 1 for few tokens)
+//                   with its lanes across the columns (coalesced 128-bit
+//                   loads, all of a 2048-column row in flight at once), a
+//                   workgroup TT tokens x 16 experts.  For a prefill an extra
+//                   row of workgroups writes x's f16 copy (prep_token): wave w
+//                   < TT takes token t0 + w.
 //                   Every product bf16 * x is exact in f64; each lane sums
 //                   its columns in f64, the lanes are added by a fixed DPP
 //                   tree, then one rounding to f32 (+ the optional logit
@@ -29,7 +30,6 @@
 namespace m1moe {
 namespace {
 
-constexpr int kTT = 4;       // tokens per logits wave and workgroup
 constexpr int kTEw = 4;      // experts per logits wave
 constexpr int kTE = 16;      // experts per logits workgroup (four waves)
 constexpr int kMaxE = 256;   // 4 logits per lane in the ranking wave
@@ -38,23 +38,23 @@ constexpr int kMaxK = 32;    // one selection per lane
 // Lane l takes columns blk * 512 + 8 l .. + 7 of each 512-column block; DB
 // blocks have their loads in flight together.  Rows past T / E are clamped
 // (loaded, never stored); columns past h are skipped.
-template <bool XBF16, int DB>
+template <bool XBF16, int DB, int TT>
 __device__ __forceinline__ void logits_wave(const RouterArgs& a, int t0, int e0, int lane,
-                                            double (&acc)[kTT][kTEw]) {
+                                            double (&acc)[TT][kTEw]) {
     const int h = a.h, nb = (h + 511) / 512;
     const uint16_t* wr[kTEw];
 #pragma unroll
     for (int j = 0; j < kTEw; ++j) wr[j] = a.router + (size_t)min(e0 + j, a.E - 1) * h;
     for (int b0 = 0; b0 < nb; b0 += DB) {
         uint4 wv[DB][kTEw];
-        float4 xv[DB][kTT][2];  // f32 x, or bf16 x in xv[][][0] as raw bits
+        float4 xv[DB][TT][2];  // f32 x, or bf16 x in xv[][][0] as raw bits
 #pragma unroll
         for (int u = 0; u < DB; ++u) {
             const int c = min((b0 + u) * 512 + lane * 8, h - 8);
 #pragma unroll
             for (int j = 0; j < kTEw; ++j) wv[u][j] = *reinterpret_cast<const uint4*>(wr[j] + c);
 #pragma unroll
-            for (int i = 0; i < kTT; ++i) {
+            for (int i = 0; i < TT; ++i) {
                 const size_t row = (size_t)min(t0 + i, a.T - 1) * h + c;
                 if (XBF16) {
                     const uint4 q = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.x) + row);
@@ -70,7 +70,7 @@ __device__ __forceinline__ void logits_wave(const RouterArgs& a, int t0, int e0,
         for (int u = 0; u < DB; ++u) {
             if ((b0 + u) * 512 + lane * 8 >= h) continue;
 #pragma unroll
-            for (int i = 0; i < kTT; ++i) {
+            for (int i = 0; i < TT; ++i) {
                 float x8[8];
                 if (XBF16) {
                     const uint4 q = __builtin_bit_cast(uint4, xv[u][i][0]);
@@ -134,29 +134,28 @@ __device__ void prep_token(const RouterArgs& a, int t, int lane) {
     if (lane == 0) a.xinv[t] = inv;
 }
 
-static_assert(kTT == 4, "one wave of the 256-thread workgroup per token");
-
+template <int TT>
 __global__ __launch_bounds__(256) void router_logits_kernel(RouterArgs a) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t0 = blockIdx.x * kTT, e0 = blockIdx.y * kTE + wave * kTEw;
+    const int t0 = blockIdx.x * TT, e0 = blockIdx.y * kTE + wave * kTEw;
     // for a prefill, an extra row of workgroups (the last) makes the f16 copy:
-    // wave w takes token t0 + w, beside the logits of the other rows
+    // wave w < TT takes token t0 + w, beside the logits of the other rows
     if (a.xq && blockIdx.y == gridDim.y - 1) {
-        prep_token(a, t0 + wave, lane);
+        if (wave < TT) prep_token(a, t0 + wave, lane);
         return;
     }
     if (e0 >= a.E) return;
-    double acc[kTT][kTEw];
+    double acc[TT][kTEw];
 #pragma unroll
-    for (int i = 0; i < kTT; ++i)
+    for (int i = 0; i < TT; ++i)
 #pragma unroll
         for (int j = 0; j < kTEw; ++j) acc[i][j] = 0.0;
     if (a.x_bf16)
-        logits_wave<true, 4>(a, t0, e0, lane, acc);
+        logits_wave<true, 4, TT>(a, t0, e0, lane, acc);
     else
-        logits_wave<false, 2>(a, t0, e0, lane, acc);
+        logits_wave<false, (TT <= 2 ? 4 : 2), TT>(a, t0, e0, lane, acc);
 #pragma unroll
-    for (int i = 0; i < kTT; ++i)
+    for (int i = 0; i < TT; ++i)
 #pragma unroll
         for (int j = 0; j < kTEw; ++j) {
             const double v = wave_sum_f64_last(acc[i][j]);  // lane 63
@@ -257,15 +256,33 @@ __global__ __launch_bounds__(256) void router_rank_kernel(RouterArgs a) {
     }
 }
 
+constexpr long kFewWorkgroups = 256;   // one per CU
+
+template <int TT>
+void launch_logits(const RouterArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL(router_logits_kernel<TT>,
+                       dim3((unsigned)((a.T + TT - 1) / TT),
+                            (unsigned)((a.E + kTE - 1) / kTE + (a.xq ? 1 : 0))),
+                       dim3(256), 0, st, a);
+}
+
 }  // namespace
 
 int launch_router_topk(const RouterArgs& a, void* stream) {
     if (a.E > kMaxE || a.K > kMaxK || a.h % 64) return (int)hipErrorInvalidValue;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(router_logits_kernel,
-                       dim3((unsigned)((a.T + kTT - 1) / kTT),
-                            (unsigned)((a.E + kTE - 1) / kTE + (a.xq ? 1 : 0))),
-                       dim3(256), 0, st, a);
+    // The fewest tokens per wave whose grid fits the CUs once: a short prompt's
+    // launch is the time of one wave (T = 37 x 64 experts x 2048 7.2 us at four,
+    // 5.2 at two, 4.7 at one; T = 128 7.2, 5.5, 6.3; T = 50 x 8 x 4096 10.6, 7.6,
+    // 6.5), a long one's the loads and conversions that more tokens share (T =
+    // 512 11.5 us at four, 13.9, 16.6; T = 1000 x 8 x 4096 15.7, 19.2, 17.6).
+    const long groups = (a.E + kTE - 1) / kTE;
+    if (a.T * groups <= kFewWorkgroups)
+        launch_logits<1>(a, st);
+    else if ((a.T + 1) / 2 * groups <= kFewWorkgroups)
+        launch_logits<2>(a, st);
+    else
+        launch_logits<4>(a, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     const dim3 g((unsigned)((a.T + 3) / 4));

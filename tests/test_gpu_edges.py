@@ -62,6 +62,43 @@ def test_rmsnorm_edges(ops_ctx, n):
         b.free()
 
 
+# ---- router -----------------------------------------------------------------------------
+
+
+@pytest.mark.parametrize("T", [1, 3, 127, 128, 129, 255, 256, 257, 511, 513])
+@pytest.mark.parametrize("name", ["tiny", "tiny_renorm"])
+def test_router_tokens_per_wave(name, T):
+    """Both sides of every tokens-per-wave rule (8 and 16 experts, one workgroup
+    row): logits bit for bit as the oracle's (f64 sums rounded once), top-K
+    exact, weights to a few f32 roundings."""
+    from cases import make_case
+    from m1moe_amd import synth
+    from m1moe_amd.engine import MoEBlock
+    c = make_case(name, seed=71)
+    try:
+        E, K = c.shape.num_experts, c.shape.top_k
+        x = c.x_bf16(T)
+        dx = c.ctx.to_device(x)
+        di, dw, dl = c.ctx.alloc(4 * T * K), c.ctx.alloc(4 * T * K), c.ctx.alloc(4 * T * E)
+        say(f"router {name} T={T}")
+        MoEBlock(c.ctx).router_topk(0, T, dx, "bf16", di, dw, dl)
+        c.ctx.sync()
+        idx, w = di.download(np.int32).reshape(T, K), dw.download(np.float32).reshape(T, K)
+        logits = dl.download(np.float32).reshape(T, E)
+        want = (synth.bf16_to_f32(x).astype(np.float64) @
+                synth.bf16_to_f32(c.routers[0]).astype(np.float64).T).astype(np.float32)
+        assert np.array_equal(logits, want)
+        order = np.argsort(-want, axis=1, kind="stable")[:, :K]
+        assert np.array_equal(idx, order)
+        p = np.exp(want.astype(np.float64) - want.max(1, keepdims=True))
+        p = np.take_along_axis(p / p.sum(1, keepdims=True), order, 1)
+        if c.shape.norm_topk_prob:
+            p /= p.sum(1, keepdims=True)
+        assert np.abs(w - p).max() < 1e-6
+    finally:
+        c.close()
+
+
 # ---- decode attention -------------------------------------------------------------------
 
 
