@@ -478,6 +478,7 @@ int32_t dec_step(m1moe_dec_t dec, const int32_t* tok_in, int32_t* tok_out, int32
         o.attn_qh = at.qh;
         o.attn_hd = hd;
         o.attn_nch = at.nch;
+        o.attn_scale = at.scale;
         o.pos = dec->pos;
         o.max_seq = at.max_seq;
         if ((rc = launched(launch_matvec_bf16(o, st), "o_proj"))) return rc;

@@ -204,6 +204,19 @@ __device__ __forceinline__ RowRef mv_row(const MvArgs& a, int row) {
 // (InferenceEngine.swift:482-488), then (norm_w) RMS-normalised
 // (Shaders.metal:96-134).  Workgroup 0 stores the un-normalised input to
 // x_copy.
+// Decode attention keeps its scores as the raw dot products q . k: a softmax
+// weight is 2^((q . k - max) unit), unit = scale log2(e).  The difference is
+// taken first, so what is rounded after the dot product is no larger than the
+// exponent itself, whatever the scores' size, and every maximum that chunks,
+// waves and lanes are merged by is a score as it was compared.  (Scaling the
+// queries first and converting the chunks' maxima to exponents of e: 16 heads
+// of 128 at 200 positions 1.65e-7 off 64 bits, 1.52e-7 now; queries eight times
+// as large 4.1e-7 and 3.4e-7; same time, 6.69 and 6.64 us.)
+constexpr float kLog2e = 1.44269504f;
+__device__ __forceinline__ float attn_weight(float diff, float unit) {
+    return __builtin_amdgcn_exp2f(diff * unit);
+}
+
 // Active chunks of a fused decode-attention launch at position p if it
 // leaves their merge to the next launch, else 0 (one chunk: the attention
 // launch writes the output itself; many: the merge stays there, where the
@@ -219,14 +232,15 @@ __device__ __forceinline__ int attn_defer_nact(int p, int max_seq, int nch, int 
 }
 
 // x[h * hd + d] of the deferred attention merge: per head M = max_c m_c,
-// x = sum_c acc_c[d] e^(m_c - M) / sum_c l_c e^(m_c - M) (chunks in order),
-// over the partials [groups][chunks][qh][hd + 2] of the attention launch.
+// f_c = attn_weight(m_c - M), x = sum_c acc_c[d] f_c / sum_c l_c f_c (chunks in
+// order), over the partials [groups][chunks][qh][hd + 2] of the attention launch.
 // Each thread takes 4 consecutive elements (one head); all of its loads are
 // issued before they are used.
 __device__ float mv_stage_attn(const MvArgs& a, int nact, float* s_x) {
     const int n4 = a.cols >> 2;
     const int hs = a.attn_hd + 2;
     const size_t cstride = (size_t)a.attn_qh * hs;
+    const float unit = a.attn_scale * kLog2e;
     float ss = 0.f;
     for (int i4 = threadIdx.x; i4 < n4; i4 += 256) {
         const int i = 4 * i4, h = i / a.attn_hd, d = i - h * a.attn_hd;
@@ -250,7 +264,7 @@ __device__ float mv_stage_attn(const MvArgs& a, int nact, float* s_x) {
 #pragma unroll
         for (int c = 0; c < kAttnDeferChunks; ++c) {
             if (c >= nact) break;
-            const float f = expf(m[c] - M);
+            const float f = attn_weight(m[c] - M, unit);
             L = fmaf(l[c], f, L);
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = fmaf(v[c][e], f, acc[e]);
@@ -638,7 +652,7 @@ __host__ __device__ constexpr bool attn_sync_fits(int nact) {
 // The synchronous merge, workgroup (g, c)'s share: outputs o0 .. o0 + S - 1 of
 // its group's QH * HD (S = ceil(QH HD / nact), o0 = c S), each taken by R
 // lanes (R S <= 256, R <= 16) that add every R-th chunk; per head M = max_c
-// m_c, f_c = e^(m_c - M), L = sum_c l_c f_c (from the chunk statistics,
+// m_c, f_c = attn_weight(m_c - M), L = sum_c l_c f_c (from the chunk statistics,
 // staged in LDS), out = sum_c acc_c f_c / L.  Every value is read until it
 // carries this launch's number (the other workgroups' stores are not
 // waited for); the waits are bounded (a timeout raises device flag 4).
@@ -696,7 +710,7 @@ __device__ void attn_merge_share(const AttnArgs& a, int g, int c, int nch, int n
         const bool on = lane < nact;
         const float m = on ? s_st[0][i][lane] : -INFINITY;
         const float mx = wave_max(m);
-        const float f = on ? expf(m - mx) : 0.f;
+        const float f = on ? attn_weight(m - mx, a.scale * kLog2e) : 0.f;
         const float l = wave_sum(on ? s_st[1][i][lane] * f : 0.f);
         if (on) s_st[0][i][lane] = f;
         if (lane == 0) s_l[i] = l;
@@ -815,7 +829,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) float s_q[QH][HD];
     __shared__ __attribute__((aligned(16))) float s_kv[2][HD];
     __shared__ __attribute__((aligned(16))) float s_acc[4][QH][HD];
-    __shared__ float s_wm[4][QH], s_wl[4][QH];     // per wave: maximum (exponent of two), sum
+    __shared__ float s_wm[4][QH], s_wl[4][QH];     // per wave: maximum, sum
     __shared__ float s_l[QH];                      // merge: sum per head
     __shared__ float s_st[2][QH][kAttnMaxChunks];  // merge: chunk max and sum
     __shared__ int s_flag;
@@ -854,6 +868,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
         seq = a.seq_len;
     }
     const bool has_new = a.fused && p < a.max_seq;  // row p comes from k_new / v_new
+    const float unit = a.scale * kLog2e;
     const int chunk = attn_chunk(seq, nch);
     const int c0 = c * chunk, c1 = min(c0 + chunk, seq);
     const int nact = (seq + chunk - 1) / chunk;  // workgroups with positions
@@ -966,13 +981,8 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
         for (int i = 0; i < QH; ++i)
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
-        // running maximum of the scores (exponents of two: the queries are scaled)
-        // and sum of this lane's position group (the same in its LP lanes)
-        const Log2Scale scaled(a.scale);
-#pragma unroll
-        for (int i = 0; i < QH; ++i)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qv[i][e] = scaled(qv[i][e]);
+        // running maximum of the scores (raw dot products) and sum of this lane's
+        // position group (the same in its LP lanes)
         float m[QH], l[QH];
 #pragma unroll
         for (int i = 0; i < QH; ++i) {
@@ -1024,14 +1034,14 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
 #pragma unroll
                 for (int it = 0; it < SB; ++it) mn = fmaxf(mn, s[it][i]);
                 const float mc = mn == -INFINITY ? 0.f : mn;
-                const float f = __builtin_amdgcn_exp2f(m[i] - mc);
+                const float f = attn_weight(m[i] - mc, unit);
                 m[i] = mn;
                 l[i] *= f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) acc[i][e] *= f;
 #pragma unroll
                 for (int it = 0; it < SB; ++it) {
-                    const float w = __builtin_amdgcn_exp2f(s[it][i] - mc);
+                    const float w = attn_weight(s[it][i] - mc, unit);
                     const float4 v0 = R.v[it][0], v1 = R.v[it][1];
                     l[i] += w;
                     acc[i][0] = fmaf(w, v0.x, acc[i][0]);
@@ -1060,7 +1070,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < QH; ++i) {
             const float M = lane_stride_max<LP>(m[i]);
-            const float f = m[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[i] - M);
+            const float f = m[i] == -INFINITY ? 0.f : attn_weight(m[i] - M, unit);
             l[i] = lane_stride_sum<LP>(l[i] * f);
             m[i] = M;
 #pragma unroll
@@ -1085,7 +1095,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
             return fmaxf(fmaxf(s_wm[0][i], s_wm[1][i]), fmaxf(s_wm[2][i], s_wm[3][i]));
         };
         auto wave_factor = [&](int w, int i, float M) {
-            return s_wm[w][i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_wm[w][i] - M);
+            return s_wm[w][i] == -INFINITY ? 0.f : attn_weight(s_wm[w][i] - M, unit);
         };
         auto head_sum = [&](int i, float M) {
             float t = 0.f;
@@ -1111,17 +1121,17 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
         // (a deferred merge reads the partials in the next launch: plain stores;
         // the synchronous merge: (launch number, value) pairs)
         const uint32_t tag = s_tag;
-        if (tid >= 256 - QH) {   // (the last wave; the chunk's maximum as an exponent of e)
+        if (tid >= 256 - QH) {   // (the last wave)
             const int i = tid - (256 - QH);
-            const float M = head_max(i), L = head_sum(i, M), Ms = M * 0.693147181f;
+            const float M = head_max(i), L = head_sum(i, M);
             if (sync) {
-                st_coh_u64(part64 + i * (HD + 2), tagged64(tag, Ms));
+                st_coh_u64(part64 + i * (HD + 2), tagged64(tag, M));
                 st_coh_u64(part64 + i * (HD + 2) + 1, tagged64(tag, L));
             } else if (defer) {
-                part[i * (HD + 2)] = Ms;
+                part[i * (HD + 2)] = M;
                 part[i * (HD + 2) + 1] = L;
             } else {
-                st_coh(part + i * (HD + 2), Ms);
+                st_coh(part + i * (HD + 2), M);
                 st_coh(part + i * (HD + 2) + 1, L);
             }
         }
@@ -1149,7 +1159,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
     }
 
     // the last workgroup of the group merges the nact partials:
-    // out = sum_c acc_c e^(m_c - M) / sum_c l_c e^(m_c - M)
+    // out = sum_c acc_c f_c / sum_c l_c f_c, f_c = attn_weight(m_c - M)
     if (!last_workgroup(a.counters + g, nch, &s_flag)) return;
     const size_t cstride = (size_t)QH * (HD + 2);
     const float* base = a.partial + (size_t)g * nch * cstride;
@@ -1194,7 +1204,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
                                  : 0.f;
         }
         if (cb == 0) {
-            // per head: M = max_c m_c, factors f_c = e^(m_c - M) (in place of
+            // per head: M = max_c m_c, factors f_c = attn_weight(m_c - M) (in place of
             // m_c), L = sum_c l_c f_c -- once per (head, chunk), not per output
 #pragma unroll
             for (int s = 0; s < kSt; ++s) {
@@ -1208,7 +1218,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
                 const bool ok = lane < nact;
                 const float m = ok ? s_st[0][i][lane] : -INFINITY;
                 const float mx = wave_max(m);
-                const float f = ok ? expf(m - mx) : 0.f;
+                const float f = ok ? attn_weight(m - mx, unit) : 0.f;
                 const float l = wave_sum(ok ? s_st[1][i][lane] * f : 0.f);
                 if (ok) s_st[0][i][lane] = f;
                 if (lane == 0) s_l[i] = l;

@@ -308,6 +308,7 @@ struct MvArgs {
     // partial buffer, the other fields its AttnArgs geometry; null: x given
     const float* attn_part;
     int32_t attn_heads, attn_qh, attn_hd, attn_nch;
+    float attn_scale;
 };
 
 // Decode attention of one query position.  Workgroup (g, c): q heads

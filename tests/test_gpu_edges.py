@@ -130,6 +130,94 @@ def test_attention_decode_chunk_edges(ops_ctx, nh, nkv, hd, sl):
         b.free()
 
 
+# queries of few bits in one dimension: with keys of 10 bits every dot product is
+# exact in f32; at head_dim 64 the scores are 300 to 500 exponents of two
+_LARGE_Q = (1920.0, 2176.0, 2304.0)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,sl", [
+    (2, 1, 64, 300), (8, 1, 64, 700), (4, 1, 128, 300), (16, 16, 64, 1000), (8, 1, 256, 700),   # merged in the launch
+    (8, 1, 256, 130), (300, 300, 64, 333)])                    # by each group's last workgroup
+def test_attention_decode_merges_large_scores(ops_ctx, nh, nkv, hd, sl):
+    """Large scores that differ from chunk to chunk by up to 12 exponents of two,
+    their dot products exact in f32: what is left is the rounding of the
+    exponents (12 x 2^-24 x ln 2), the hardware exp2 (one ulp), the f32 numerators
+    and their sums, 5e-7 in all.  Scores or maxima rounded at their own size
+    (2^-25 of 400) are off by several 1e-6."""
+    ctx, ops = ops_ctx
+    rng = np.random.default_rng(nh + sl)
+    q = np.zeros((nh, hd), np.float32)
+    q[:, 5] = np.array(_LARGE_Q)[np.arange(nh) % 3]
+    n = q[:, 5].astype(np.float64) / np.sqrt(hd) * np.log2(np.e)
+    p = np.arange(sl)
+    kc = rng.normal(0, 1, (sl, nkv, hd)).astype(np.float32)    # (the other dims of q are 0)
+    kc[:, :, 5] = (1 - (p * 7 % 16 + 3 * (p // 64) % 16) / 1024)[:, None]
+    vc = rng.normal(0, 1, (sl, nkv, hd)).astype(np.float32)
+    e = n[:, None] * kc[:, 0, 5].astype(np.float64)
+    w = np.exp2(e - e.max(1, keepdims=True))
+    w /= w.sum(1, keepdims=True)
+    want = np.stack([w[i] @ vc[:, i * nkv // nh].astype(np.float64) for i in range(nh)])
+    dq, dk, dv, dout = ctx.to_device(q), ctx.to_device(kc), ctx.to_device(vc), ctx.alloc(4 * nh * hd)
+    say(f"attention large scores nh={nh} nkv={nkv} hd={hd} seq={sl}")
+    ops.attention_decode(dq, dk, dv, dout, nh, nkv, hd, sl)
+    ctx.sync()
+    rel = rel_l2(dout.download(np.float32).reshape(nh, hd), want)
+    say(f"rel L2 {rel:.2e}")
+    assert rel < 5e-7
+    for b in (dq, dk, dv, dout):
+        b.free()
+
+
+def test_decoder_step_merges_large_scores():
+    """The same through a decoder step, 5 chunks (merged by o_proj while it
+    stages its input) and 10 (in the attention launch): embeddings of +-1 and
+    eps 0 make the projections' input exactly +-1, a RoPE base of 1e30 leaves the
+    last pair of a head unrotated, zeroed experts leave the residual.  Bound: the
+    attention's 5e-7 and the f32 sums of v, o_proj, norm and lm_head."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import _lib, synth
+    from m1moe_amd.synth import bf16_to_f32
+    wl = synth.DecoderWorkload("wide", synth.CONFIGS["tiny"], 1, 300, 2, 1, 64, 1e30, False, 8, 8,
+                               rms_eps=0.0)
+    p = Pair(wl, seed=64, max_seq=700)
+    try:
+        _zero_experts(p)
+        h, hd, D = 128, 64, 31
+        rng = np.random.default_rng(64)
+        emb = rng.choice([-1.0, 1.0], (wl.vocab, h))
+        emb[:, :4] = 1
+        emb[:, 4:10] = 1 - 2 * (np.arange(wl.vocab)[:, None] >> np.arange(6) & 1)
+        wq, wk = np.zeros((2 * hd, h)), np.zeros((hd, h))
+        wq[[D, hd + D], 0] = _LARGE_Q[1:]
+        wk[D, 3] = 1 - 2.0 ** -4
+        wk[D, 4:10] = 2.0 ** -np.arange(10, 4, -1)   # (keys of 10 bits)
+        ones, val = np.ones(h), {}
+        for which, a in ((_lib.W_EMBED, emb), (_lib.W_IN_NORM, ones), (_lib.W_POST_NORM, ones),
+                         (_lib.W_FINAL_NORM, ones), (_lib.W_Q, wq), (_lib.W_K, wk),
+                         (_lib.W_V, rng.normal(0, 1, (hd, h))), (_lib.W_O, rng.normal(0, 0.1, (h, 2 * hd))),
+                         (_lib.W_LM_HEAD, rng.normal(0, 0.1, (wl.vocab, h)))):
+            p.dec.upload(which, 0, bf16(a))
+            val[which] = bf16_to_f32(bf16(a)).astype(np.float64)
+        toks = np.array([i * 7 % 16 + 3 * (i // 64) % 16 + 64 * (i % 4) for i in range(640)], np.int32)
+        for n in (300, 620):
+            p.dec.reset()
+            p.dec.prefill(toks[:n - 1])
+            say(f"step {n}")
+            _, got = p.dec.forward(int(toks[n - 1]), return_logits=True)
+            x = val[_lib.W_EMBED][toks[:n]]
+            k, v = x @ val[_lib.W_K].T, x @ val[_lib.W_V].T
+            q = (val[_lib.W_Q] @ x[-1]).reshape(2, hd)
+            e = q @ k.T / 8 * np.log2(np.e)
+            w = np.exp2(e - e.max(1, keepdims=True))
+            att = (w / w.sum(1, keepdims=True)) @ v
+            y = x[-1] + val[_lib.W_O] @ att.reshape(-1)
+            rel = rel_l2(got, val[_lib.W_LM_HEAD] @ (y / np.sqrt((y * y).mean())))
+            say(f"rel L2 {rel:.2e}")
+            assert rel < 1e-6
+    finally:
+        p.close()
+
+
 def test_decoder_steps_in_a_long_cache():
     """A cache of 5000 positions shared by 16 workgroups per head: the chunk
     grows with the position (64 up to 1024 positions, then more), the
