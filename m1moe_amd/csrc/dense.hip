@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "device.hpp"
 #include "internal.hpp"
@@ -814,8 +815,15 @@ __host__ __device__ constexpr int attn_sb() {
     return V == 0 ? HD / 32 : V == 2 ? HD / 32 + 1 : QH == 8 ? 2 : 4;
 }
 
+// Workgroups per CU that the registers leave room for: one where eight heads of
+// 256 take a whole quarter of a chunk as one batch.
 template <int HD, int QH, int V>
-__global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
+constexpr int attn_wgs() {
+    return QH == 8 && HD == 256 && V == 0 ? 1 : 2;
+}
+
+template <int HD, int QH, int V>
+__global__ __launch_bounds__(256, (attn_wgs<HD, QH, V>())) void attn_kernel(AttnArgs a) {
     if (blockIdx.z) {
         attn_prefetch(a);
         return;
@@ -989,10 +997,12 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
             m[i] = -INFINITY;
             l[i] = 0.f;
         }
-        auto batch = [&](int p0, KVRows& R) {
-            if (mine_new && p >= p0 && p < p0 + BP) {   // (uniform)
+        // the first `count` loads of a batch at p0
+        auto batch = [&](int p0, KVRows& R, auto count) {
+            constexpr int NB = decltype(count)::value;
+            if (mine_new && p >= p0 && p < p0 + NB * PPI) {   // (uniform)
 #pragma unroll
-                for (int it = 0; it < SB; ++it) {
+                for (int it = 0; it < NB; ++it) {
                     if (p0 + it * PPI + pg != p) continue;
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
@@ -1002,9 +1012,9 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
                 }
             }
             // scores (attnScores, Shaders.metal:209-243)
-            float s[SB][QH];
+            float s[NB][QH];
 #pragma unroll
-            for (int it = 0; it < SB; ++it)
+            for (int it = 0; it < NB; ++it)
 #pragma unroll
                 for (int i = 0; i < QH; ++i) {
                     const float4 k0 = R.k[it][0], k1 = R.k[it][1];
@@ -1018,9 +1028,9 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
                     d = fmaf(qv[i][7], k1.w, d);
                     s[it][i] = lane_group_sum<LP>(d);
                 }
-            if (w1 - p0 < BP) {   // (uniform) positions past the wave's: weight 0 on zeros
+            if (w1 - p0 < NB * PPI) {   // (uniform) positions past the wave's: weight 0 on zeros
 #pragma unroll
-                for (int it = 0; it < SB; ++it)
+                for (int it = 0; it < NB; ++it)
                     if (p0 + it * PPI + pg >= w1) {
                         R.v[it][0] = R.v[it][1] = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1032,7 +1042,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
             for (int i = 0; i < QH; ++i) {
                 float mn = m[i];
 #pragma unroll
-                for (int it = 0; it < SB; ++it) mn = fmaxf(mn, s[it][i]);
+                for (int it = 0; it < NB; ++it) mn = fmaxf(mn, s[it][i]);
                 const float mc = mn == -INFINITY ? 0.f : mn;
                 const float f = attn_weight(m[i] - mc, unit);
                 m[i] = mn;
@@ -1040,7 +1050,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) acc[i][e] *= f;
 #pragma unroll
-                for (int it = 0; it < SB; ++it) {
+                for (int it = 0; it < NB; ++it) {
                     const float w = attn_weight(s[it][i] - mc, unit);
                     const float4 v0 = R.v[it][0], v1 = R.v[it][1];
                     l[i] += w;
@@ -1057,14 +1067,18 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
         };
         if (TWO) {
             for (int p0 = w0; p0 < w1; p0 += 8 * BP) {
-                batch(p0, A);
+                batch(p0, A, std::integral_constant<int, SB>{});
                 if (p0 + 4 * BP >= w1) break;
                 load_rows(p0 + 8 * BP, A);
-                batch(p0 + 4 * BP, B);
+                batch(p0 + 4 * BP, B, std::integral_constant<int, SB>{});
                 load_rows(p0 + 12 * BP, B);
             }
+        } else if (QH == 8 && HD != 64 && w1 - w0 <= SB / 2 * PPI) {
+            // (short chunks: half the loads' worth of arithmetic, 17 positions of 8 q / 1
+            // kv head of 128 8.95 -> 7.6 us; fewer heads have less of it to leave out)
+            if (w0 < w1) batch(w0, A, std::integral_constant<int, SB / 2>{});
         } else if (w0 < w1) {
-            batch(w0, A);
+            batch(w0, A, std::integral_constant<int, SB>{});
         }
         // the wave's position groups, then (in LDS) its partial
 #pragma unroll
@@ -1340,12 +1354,10 @@ int launch_mv(const MvArgs& a, hipStream_t st) {
 
 // The kernel's V for chunks of at most attn_chunk(max_seq, nch) positions (a
 // launch over fewer positions has no longer ones): one batch per wave where a
-// quarter of the chunk fits it.  Eight heads' registers leave that to head_dim
-// 64 (8 q / 1 kv head of 64, 130 positions: 12.0 us with batches of four loads,
-// 11.1 with two).
+// quarter of the chunk fits it (8 q / 1 kv head at 130 positions, batches of two
+// loads in flight -> one batch: head_dim 128 14.0 -> 12.8 us, 256 17.8 -> 16.6).
 int attn_variant(int head_dim, int qh, int max_seq, int nch) {
     const int n = attn_chunk(max_seq, nch);
-    if (qh == 8 && head_dim != 64) return 1;
     if (n <= 64) return 0;
     return head_dim != 256 && n <= (head_dim == 64 ? 96 : 80) ? 2 : 1;
 }
@@ -1356,12 +1368,7 @@ int launch_attn_v(const AttnArgs& a, dim3 grid, hipStream_t st) {
         case 1: hipLaunchKernelGGL((attn_kernel<HD, 1, V>), grid, dim3(256), 0, st, a); break;
         case 2: hipLaunchKernelGGL((attn_kernel<HD, 2, V>), grid, dim3(256), 0, st, a); break;
         case 4: hipLaunchKernelGGL((attn_kernel<HD, 4, V>), grid, dim3(256), 0, st, a); break;
-        case 8:
-            if constexpr (V == 1 || HD == 64) {
-                hipLaunchKernelGGL((attn_kernel<HD, 8, V>), grid, dim3(256), 0, st, a);
-                break;
-            }
-            return (int)hipErrorInvalidValue;
+        case 8: hipLaunchKernelGGL((attn_kernel<HD, 8, V>), grid, dim3(256), 0, st, a); break;
         default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();
@@ -1437,10 +1444,7 @@ int attn_occupancy_v(int qh) {
         case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 1, V>, 256, 0); break;
         case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 2, V>, 256, 0); break;
         case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 4, V>, 256, 0); break;
-        case 8:
-            if constexpr (V == 1 || HD == 64)
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 8, V>, 256, 0);
-            break;
+        case 8: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_kernel<HD, 8, V>, 256, 0); break;
         default: break;
     }
     return e == hipSuccess ? n : 0;

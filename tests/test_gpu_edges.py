@@ -109,7 +109,10 @@ def test_router_tokens_per_wave(name, T):
     (64, 64, 128, 255), (64, 64, 128, 320), (64, 64, 128, 321), (64, 64, 256, 256),
     (64, 64, 256, 259), (64, 8, 64, 2049), (64, 8, 128, 130), (64, 8, 128, 8191),
     # one position past a chunk, past a wave's batch; more groups than CUs
-    (32, 8, 128, 65), (32, 8, 128, 17), (24, 8, 64, 9), (300, 300, 64, 333), (2, 2, 256, 2)])
+    (32, 8, 128, 65), (32, 8, 128, 17), (24, 8, 64, 9), (300, 300, 64, 333), (2, 2, 256, 2),
+    # eight heads per group: half a batch per wave, a whole one, the larger one
+    (8, 1, 128, 1), (8, 1, 128, 32), (8, 1, 128, 33), (64, 8, 128, 2049), (64, 8, 128, 2560),
+    (8, 1, 256, 31), (8, 1, 256, 33), (8, 1, 256, 64), (16, 2, 256, 129)])
 def test_attention_decode_chunk_edges(ops_ctx, nh, nkv, hd, sl):
     """f32 sums of at most 8191 terms against the oracle's f64: 1e-6 (2e-7
     seen), for lengths around every batch and chunk rule; the last V row is
@@ -240,6 +243,32 @@ def test_decoder_steps_in_a_long_cache():
                 _, w_lg = p.orc.step(int(t))
                 assert rel_l2(g_lg, w_lg) < 1e-5
             off += steps
+    finally:
+        p.close()
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_decoder_steps_eight_heads_per_group(hd):
+    """Steps of 8 q heads over one kv head at the first positions, around the end
+    of half a wave's batch, of a batch and of a chunk, and over several chunks."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    wl = synth.DecoderWorkload("eight", synth.CONFIGS["tiny_renorm"], 1, 300, 8, 1, hd, 1e4, True, 8, 8)
+    p = Pair(wl, seed=65, max_seq=300)
+    try:
+        _zero_experts(p)
+        toks = synth.prompt_tokens(wl, 9, 300)
+        at = 0
+        for stop, steps in ((3, 2), (31, 3), (63, 3), (128, 2), (255, 3)):
+            say(f"prefill {at} .. {stop}, then {steps} steps")
+            p.dec.prefill(toks[at:stop])
+            for t in toks[at:stop]:
+                p.orc.step(int(t))
+            for t in toks[stop:stop + steps]:
+                _, g_lg = p.dec.forward(int(t), return_logits=True)
+                _, w_lg = p.orc.step(int(t))
+                assert rel_l2(g_lg, w_lg) < 1e-5
+            at = stop + steps
     finally:
         p.close()
 
