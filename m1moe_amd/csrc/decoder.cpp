@@ -212,7 +212,11 @@ int32_t m1moe_attention_decode(m1moe_ctx_t ctx, const float* d_q, const float* d
     a.qh = attention_qh(num_heads / num_kv_heads);
     a.cus = ctx->cus;
     a.nch = attention_chunks(seq_len, num_heads / a.qh, a.cus);
-    if ((rc = ensure_attn_scratch(ctx, attention_partial_floats(num_heads, head_dim, a.nch)))) return rc;
+    // (for the most chunks any head count has over these positions: the scratch
+    // is the context's, and a shape that a graph is captured with may follow
+    // another one of as many heads and positions)
+    const int32_t most = attention_max_chunks(seq_len);
+    if ((rc = ensure_attn_scratch(ctx, attention_partial_floats(num_heads, head_dim, most)))) return rc;
     a.fused = 0;
     a.q = d_q;
     a.kcache = const_cast<float*>(d_kcache);  // read only when fused = 0

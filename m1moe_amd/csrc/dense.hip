@@ -1420,13 +1420,17 @@ int attention_qh(int hpkv) {
     return 1;
 }
 
+int attention_max_chunks(int max_positions) {
+    return std::min(kAttnMaxChunks, (max_positions + kAttnChunk - 1) / kAttnChunk);
+}
+
 // One workgroup per 64 positions while the grid fits the CUs once; above, the
 // positions shared evenly by as many workgroups as there are CUs (the waves
 // stream their rows without waiting for one another, so a second workgroup
 // on some CUs only unbalances them: 32 q / 8 kv heads, 5003 positions, 30.6 us
 // as 320 workgroups of 128 positions, 16.9 as 256 of 157).
 int attention_chunks(int max_positions, int groups, int cus) {
-    const int n = std::min(kAttnMaxChunks, (max_positions + kAttnChunk - 1) / kAttnChunk);
+    const int n = attention_max_chunks(max_positions);
     const int per = groups > 0 ? cus / groups : 0;   // workgroups per group on the CUs
     return (long)groups * n <= cus || per < 1 ? n : std::min(n, per);
 }

@@ -460,6 +460,7 @@ int attention_qh(int hpkv);
 // (num_heads / qh) and cus compute units: one per kAttnChunk positions while
 // they fit the CUs, then as many as fill the CUs once; at most kAttnMaxChunks.
 int attention_chunks(int max_positions, int groups, int cus);
+int attention_max_chunks(int max_positions);   // the most it gives, for any groups
 // Positions per workgroup of a launch over `positions` with nch workgroups per
 // group.
 M1MOE_HD inline int attn_chunk(int positions, int nch) {

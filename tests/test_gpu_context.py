@@ -118,6 +118,38 @@ def test_graph_refused_after_scratch_growth():
         c.close()
 
 
+def test_attention_capture_after_another_head_count():
+    """The attention scratch that one call made covers every other grouping of
+    as many heads over as many positions: the first call of 32 q / 4 kv heads is
+    captured (a graph may not grow scratch), and a graph of the 32-head form
+    stays valid after it."""
+    from m1moe_amd.decoder import DenseOps
+    ctx = m.HIPContext(m.make_shape(128, 8, 2, 64, 64))
+    try:
+        ops, rng, nh, hd, sl = DenseOps(ctx), np.random.default_rng(5), 32, 64, 1100
+        dq, dk, dv = (ctx.to_device(rng.normal(0, 1, s).astype(np.float32))
+                      for s in ((nh, hd), (sl, nh, hd), (sl, nh, hd)))
+        out = ctx.alloc(4 * nh * hd)
+        ops.attention_decode(dq, dk, dv, out, nh, nh, hd, sl)
+        graphs = []
+        for kv in (4, nh):
+            ctx.graph_begin()
+            try:
+                ops.attention_decode(dq, dk, dv, out, nh, kv, hd, sl)
+            finally:
+                graphs.append(ctx.graph_end())
+        for kv, g in list(zip((4, nh), graphs)) * 2:
+            say(f"replay kv={kv}")
+            g.launch()
+            ctx.sync()
+            got = out.download(np.float32).copy()
+            ops.attention_decode(dq, dk, dv, out, nh, kv, hd, sl)
+            ctx.sync()
+            assert np.array_equal(got, out.download(np.float32))
+    finally:
+        ctx.close()
+
+
 def test_upload_refuses_non_finite_scale():
     shape = synth.CONFIGS["tiny"].shape(1)
     img = synth.layer_image(shape, 41, 0)
