@@ -39,7 +39,7 @@ int32_t ensure_attn_scratch(m1moe_ctx_t ctx, uint64_t floats) {
     if (!ctx->attn_cnt) {
         int32_t rc = device_alloc((void**)&ctx->attn_cnt, kAttnCntWords * 4, "attention counters");
         if (rc) return rc;
-        HIP_TRY(hipMemset(ctx->attn_cnt, 0, kAttnCntWords * 4));
+        HIP_TRY(hipMemsetAsync(ctx->attn_cnt, 0, kAttnCntWords * 4, ctx->stream));
     }
     if (floats <= ctx->attn_part_floats) return M1MOE_OK;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -50,8 +50,10 @@ int32_t ensure_attn_scratch(m1moe_ctx_t ctx, uint64_t floats) {
     int32_t rc = device_alloc((void**)&ctx->attn_part, floats * 4, "attention scratch");
     if (rc) return rc;
     // (zeroed: the synchronous merge accepts a value carrying the current
-    // launch number, and reused device memory may hold one)
-    HIP_TRY(hipMemset(ctx->attn_part, 0, floats * 4));
+    // launch number, and reused device memory may hold one; on the launches' own
+    // stream: it does not wait for the null stream, where a memset may still run
+    // while the first launch stores its partials, whose merge then times out)
+    HIP_TRY(hipMemsetAsync(ctx->attn_part, 0, floats * 4, ctx->stream));
     ctx->attn_part_floats = floats;
     return M1MOE_OK;
 }
@@ -325,9 +327,9 @@ int32_t m1moe_dec_create(m1moe_ctx_t moe, const m1moe_dec_shape* s, m1moe_dec_t*
     }
     // (the partials are zeroed: the synchronous merge accepts a value by its
     // launch number, which starts at 1, and reused device memory may hold any)
-    if (hipMemset(d->pos, 0, 16) != hipSuccess ||
-        hipMemset(d->cnt, 0, dec_cnt_words(s->num_heads) * 4) != hipSuccess ||
-        hipMemset(d->part, 0, part * 4) != hipSuccess ||
+    if (hipMemsetAsync(d->pos, 0, 16, moe->stream) != hipSuccess ||
+        hipMemsetAsync(d->cnt, 0, dec_cnt_words(s->num_heads) * 4, moe->stream) != hipSuccess ||
+        hipMemsetAsync(d->part, 0, part * 4, moe->stream) != hipSuccess ||
         launch_rope_table(d->rope, s->max_seq, s->head_dim, s->rope_theta, moe->stream) != 0 ||
         hipStreamSynchronize(moe->stream) != hipSuccess) {
         m1moe_dec_destroy(d);

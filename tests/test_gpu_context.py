@@ -150,6 +150,31 @@ def test_attention_capture_after_another_head_count():
         ctx.close()
 
 
+def test_attention_right_after_scratch_growth():
+    """The first call over more positions allocates and zeroes its partials and
+    launches at once: the zeroes must be in before the kernel's own values (its
+    merge waits for those, and a lost one ends in a time-out at the sync)."""
+    from m1moe_amd.decoder import DenseOps
+    rng, nh, hd, most = np.random.default_rng(6), 8, 128, 6000
+    for rep in range(3):
+        ctx = m.HIPContext(m.make_shape(128, 8, 2, 64, 64))
+        try:
+            ops = DenseOps(ctx)
+            dq, dk, dv = (ctx.to_device(rng.normal(0, 1, s).astype(np.float32))
+                          for s in ((nh, hd), (most, nh, hd), (most, nh, hd)))
+            out = ctx.alloc(4 * nh * hd)
+            for sl in (130, 600, 1100, 1500, 2000, 4100, most):
+                say(f"context {rep}, {sl} positions")
+                got = []
+                for _ in range(2):
+                    ops.attention_decode(dq, dk, dv, out, nh, nh, hd, sl)
+                    ctx.sync()
+                    got.append(out.download(np.float32).copy())
+                assert np.array_equal(*got)
+        finally:
+            ctx.close()
+
+
 def test_upload_refuses_non_finite_scale():
     shape = synth.CONFIGS["tiny"].shape(1)
     img = synth.layer_image(shape, 41, 0)
