@@ -213,7 +213,7 @@ int32_t m1moe_attention_decode(m1moe_ctx_t ctx, const float* d_q, const float* d
     AttnArgs a{};
     a.qh = attention_qh(num_heads / num_kv_heads);
     a.cus = ctx->cus;
-    a.nch = attention_chunks(seq_len, num_heads / a.qh, a.cus);
+    a.split = attention_split(seq_len, num_heads / a.qh, a.cus, a.qh, head_dim);
     // (for the most chunks any head count has over these positions: the scratch
     // is the context's, and a shape that a graph is captured with may follow
     // another one of as many heads and positions)
@@ -292,9 +292,9 @@ int32_t m1moe_dec_create(m1moe_ctx_t moe, const m1moe_dec_shape* s, m1moe_dec_t*
     d->loaded.assign((size_t)kNumW * d->L, false);
     const uint64_t h = d->h, L = d->L, V = s->vocab, qd = d->qd, kvd = d->kvd, hd = s->head_dim;
     const uint64_t ms = s->max_seq;
-    const int32_t groups = s->num_heads / attention_qh(s->num_heads / s->num_kv_heads);
+    const int32_t qh = attention_qh(s->num_heads / s->num_kv_heads);
     const uint64_t part = (uint64_t)attention_partial_floats(
-        s->num_heads, s->head_dim, attention_chunks(s->max_seq, groups, moe->cus));
+        s->num_heads, s->head_dim, attention_split(s->max_seq, s->num_heads / qh, moe->cus, qh, s->head_dim).nch);
     if ((rc = dec_alloc(d, (void**)&d->embed, V * h * 2, "embedding")) ||
         (rc = dec_alloc(d, (void**)&d->lm_head, V * h * 2, "lm_head")) ||
         (rc = dec_alloc(d, (void**)&d->final_norm, h * 2, "final norm")) ||
@@ -425,7 +425,7 @@ int32_t dec_step(m1moe_dec_t dec, const int32_t* tok_in, int32_t* tok_out, int32
     at.head_dim = hd;
     at.qh = attention_qh(at.hpkv);
     at.cus = ctx->cus;
-    at.nch = attention_chunks(dec->sh.max_seq, at.num_heads / at.qh, at.cus);
+    at.split = attention_split(dec->sh.max_seq, at.num_heads / at.qh, at.cus, at.qh, hd);
     at.kv_pos = kvd;
     at.kv_head = hd;
     at.scale = 1.0f / sqrtf((float)hd);
@@ -438,7 +438,7 @@ int32_t dec_step(m1moe_dec_t dec, const int32_t* tok_in, int32_t* tok_out, int32
     at.rope = dec->rope;
     // short contexts: o_proj merges the attention partials while staging its
     // input (only a staged input can: q widths up to kMvStageMax)
-    at.defer = qd <= kMvStageMax ? 1 : 0;
+    at.defer = qd <= kMvStageMax && at.split.one == kAttnChunk ? 1 : 0;
     const uint64_t cache_layer = (uint64_t)dec->sh.max_seq * kvd;
     for (int l = 0; l < dec->L; ++l) {
         // input RMSNorm and q/k/v in one launch (InferenceEngine.swift:177-192); layer 0
@@ -483,7 +483,7 @@ int32_t dec_step(m1moe_dec_t dec, const int32_t* tok_in, int32_t* tok_out, int32
         o.attn_heads = at.num_heads;
         o.attn_qh = at.qh;
         o.attn_hd = hd;
-        o.attn_nch = at.nch;
+        o.attn_nch = at.split.nch;
         o.attn_scale = at.scale;
         o.pos = dec->pos;
         o.max_seq = at.max_seq;

@@ -834,6 +834,11 @@ __global__ __launch_bounds__(256, (attn_wgs<HD, QH, V>())) void attn_kernel(Attn
     constexpr int SB = attn_sb<HD, QH, V>();   // loads per batch
     constexpr int BP = SB * PPI;               // positions per batch
     constexpr int HALF = HD / 2;
+    // a wave with at most half a batch of positions walks half the loads' worth of
+    // arithmetic (17 positions of 8 q / 1 kv head of 128 8.95 -> 7.6 us; the early
+    // positions of a long cache, 16 q / 4 kv heads of 64, 4 layers, 119 -> 115 us a
+    // step; where there is less of it to leave out the branch costs as much)
+    constexpr bool SHORT = TWO ? HD == 64 && QH < 8 : QH == 8 && HD != 64;
     __shared__ __attribute__((aligned(16))) float s_q[QH][HD];
     __shared__ __attribute__((aligned(16))) float s_kv[2][HD];
     __shared__ __attribute__((aligned(16))) float s_acc[4][QH][HD];
@@ -877,7 +882,7 @@ __global__ __launch_bounds__(256, (attn_wgs<HD, QH, V>())) void attn_kernel(Attn
     }
     const bool has_new = a.fused && p < a.max_seq;  // row p comes from k_new / v_new
     const float unit = a.scale * kLog2e;
-    const int chunk = attn_chunk(seq, nch);
+    const int chunk = seq <= a.split.one ? a.split.one : attn_chunk(seq, nch);
     const int c0 = c * chunk, c1 = min(c0 + chunk, seq);
     const int nact = (seq + chunk - 1) / chunk;  // workgroups with positions
     const bool defer = a.defer && attn_defer_nact(p, a.max_seq, nch, a.num_heads) > 0;
@@ -911,7 +916,7 @@ __global__ __launch_bounds__(256, (attn_wgs<HD, QH, V>())) void attn_kernel(Attn
             }
         };
         load_rows(w0, A);
-        if (TWO) load_rows(w0 + 4 * BP, B);
+        if (TWO && (!SHORT || w0 + 4 * BP < w1)) load_rows(w0 + 4 * BP, B);   // (uniform)
         // keep both batches' loads here (the compiler may otherwise sink the
         // second to its first use, a memory round trip later)
         asm volatile("" ::: "memory");
@@ -997,7 +1002,6 @@ __global__ __launch_bounds__(256, (attn_wgs<HD, QH, V>())) void attn_kernel(Attn
             m[i] = -INFINITY;
             l[i] = 0.f;
         }
-        // the first `count` loads of a batch at p0
         auto batch = [&](int p0, KVRows& R, auto count) {
             constexpr int NB = decltype(count)::value;
             if (mine_new && p >= p0 && p < p0 + NB * PPI) {   // (uniform)
@@ -1065,20 +1069,20 @@ __global__ __launch_bounds__(256, (attn_wgs<HD, QH, V>())) void attn_kernel(Attn
                 }
             }
         };
-        if (TWO) {
+        typedef std::integral_constant<int, SB> Whole;
+        typedef std::integral_constant<int, SB / 2> Half;
+        if (SHORT && w1 - w0 <= SB / 2 * PPI) {
+            if (w0 < w1) batch(w0, A, Half{});
+        } else if (TWO) {
             for (int p0 = w0; p0 < w1; p0 += 8 * BP) {
-                batch(p0, A, std::integral_constant<int, SB>{});
+                batch(p0, A, Whole{});
                 if (p0 + 4 * BP >= w1) break;
                 load_rows(p0 + 8 * BP, A);
-                batch(p0 + 4 * BP, B, std::integral_constant<int, SB>{});
+                batch(p0 + 4 * BP, B, Whole{});
                 load_rows(p0 + 12 * BP, B);
             }
-        } else if (QH == 8 && HD != 64 && w1 - w0 <= SB / 2 * PPI) {
-            // (short chunks: half the loads' worth of arithmetic, 17 positions of 8 q / 1
-            // kv head of 128 8.95 -> 7.6 us; fewer heads have less of it to leave out)
-            if (w0 < w1) batch(w0, A, std::integral_constant<int, SB / 2>{});
         } else if (w0 < w1) {
-            batch(w0, A, std::integral_constant<int, SB>{});
+            batch(w0, A, Whole{});
         }
         // the wave's position groups, then (in LDS) its partial
 #pragma unroll
@@ -1352,14 +1356,16 @@ int launch_mv(const MvArgs& a, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-// The kernel's V for chunks of at most attn_chunk(max_seq, nch) positions (a
-// launch over fewer positions has no longer ones): one batch per wave where a
+// The kernel's V for chunks of at most n positions: one batch per wave where a
 // quarter of the chunk fits it (8 q / 1 kv head at 130 positions, batches of two
 // loads in flight -> one batch: head_dim 128 14.0 -> 12.8 us, 256 17.8 -> 16.6).
-int attn_variant(int head_dim, int qh, int max_seq, int nch) {
-    const int n = attn_chunk(max_seq, nch);
+int attn_variant(int head_dim, int n) {
     if (n <= 64) return 0;
     return head_dim != 256 && n <= (head_dim == 64 ? 96 : 80) ? 2 : 1;
+}
+// (a launch over fewer positions than max_seq has no longer chunks)
+int attn_variant(const AttnArgs& a) {
+    return attn_variant(a.head_dim, std::max(attn_chunk(a.max_seq, a.split.nch), a.split.one));
 }
 
 template <int HD, int V>
@@ -1429,10 +1435,37 @@ int attention_max_chunks(int max_positions) {
 // stream their rows without waiting for one another, so a second workgroup
 // on some CUs only unbalances them: 32 q / 8 kv heads, 5003 positions, 30.6 us
 // as 320 workgroups of 128 positions, 16.9 as 256 of 157).
-int attention_chunks(int max_positions, int groups, int cus) {
-    const int n = attention_max_chunks(max_positions);
-    const int per = groups > 0 ? cus / groups : 0;   // workgroups per group on the CUs
-    return (long)groups * n <= cus || per < 1 ? n : std::min(n, per);
+//
+// Where that makes long chunks (V 1), a group's first positions stay one
+// workgroup's, as many as it walks in less time than a merge takes; few workgroups
+// per group gain less by sharing, many heads x dims per position cost more (us as
+// one workgroup / as shared: 86 heads of 128 at 257 positions 9.1 / 9.6 .. 11.2, at
+// 700 15.3 / 17.9; 70 of 64 at 257 6.8 / 8.4, at 500 8.4 / 9.7; a decoder step of 4
+// layers with 32 heads of 64 at position 100 of a long cache 116 / 125; 8 q / 1 kv
+// head of 128 147 / 139).
+//
+// More groups than CUs: up to 256 positions need no merge (257 heads of 128 at 192:
+// 12.6 / 12.4 .. 15.5, at 256 16.0 / 17.4); above, short chunks in the kernel's light
+// forms (300 heads of 64 at 2000: 58.9 as 32 chunks, 67 .. 70 as 8 .. 16), then chunks
+// of at least 256 (257 heads of 128 at 2000: 98 as 8, 106 as 16 or 32; at 4100 189 as
+// 16, 204 as 64).
+AttnSplit attention_split(int max_positions, int groups, int cus, int qh, int head_dim) {
+    const int n = attention_max_chunks(max_positions), per = cus / groups;   // workgroups per group on the CUs
+    if (per < 1) {
+        if (n <= 4) return {1, kAttnChunk};
+        const int light = std::min(n, head_dim == 64 ? 32 : 16);
+        if (attn_variant(head_dim, attn_chunk(max_positions, light)) != 1) return {light, kAttnChunk};
+        return {std::min((max_positions + 255) / 256, 16), kAttnChunk};
+    }
+    const int nch = groups * n <= cus ? n : std::min(n, per), dims = qh * head_dim;
+    int one = kAttnChunk;
+    if (attn_variant(head_dim, attn_chunk(max_positions, nch)) == 1) {
+        if (per <= 12 && dims <= 256)
+            one = per > 4 ? 256 : dims <= 64 ? 512 : per > 2 ? 256 : 320;
+        else if (per <= 16 && dims <= 512 && groups * qh > 24)   // (fewer heads leave their merge to o_proj)
+            one = 128;
+    }
+    return {max_positions <= one ? 1 : nch, one};
 }
 
 int attention_partial_floats(int num_heads, int head_dim, int nch) {
@@ -1478,17 +1511,20 @@ int attn_blocks_per_cu(int hd, int qh, int v) {
 }
 }  // namespace
 
+// (not with more groups than CUs: workgroups that wait hold the CUs that others
+// could stream on, 257 heads of 64 at 257 positions 12.9 us, 9.3 merged by each
+// group's last workgroup)
 bool attention_grid_fits(const AttnArgs& a) {
-    if (a.qh <= 0 || a.qh > 8 || a.cus <= 0) return false;
-    const int64_t grid = (int64_t)(a.num_heads / a.qh) * a.nch;
-    const int v = attn_variant(a.head_dim, a.qh, a.max_seq, a.nch);
+    if (a.qh <= 0 || a.qh > 8 || a.cus < a.num_heads / a.qh) return false;
+    const int64_t grid = (int64_t)(a.num_heads / a.qh) * a.split.nch;
+    const int v = attn_variant(a);
     return (int64_t)attn_blocks_per_cu(a.head_dim, a.qh, v) * a.cus >= grid;
 }
 
 int launch_attention(const AttnArgs& a, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (a.qh <= 0 || a.num_heads % a.qh || a.hpkv % a.qh ||
-        a.nch != attention_chunks(a.max_seq, a.num_heads / a.qh, a.cus))
+        a.split.nch <= 0 || a.split.nch > kAttnMaxChunks || a.split.one < kAttnChunk)
         return (int)hipErrorInvalidValue;
     if (a.kv_pos <= 0 || a.kv_head <= 0) return (int)hipErrorInvalidValue;
     if (a.sync_merge && !(a.gen && a.fin && attention_grid_fits(a))) return (int)hipErrorInvalidValue;
@@ -1497,10 +1533,10 @@ int launch_attention(const AttnArgs& a, void* stream) {
         return (int)hipErrorInvalidValue;
     // (the prefetch planes only where the attention leaves most CUs idle: on a
     // full grid they compete with it, cfg4 2615 -> 2670 us per token)
-    const unsigned gx = (unsigned)(a.num_heads / a.qh), gy = (unsigned)a.nch;
+    const unsigned gx = (unsigned)(a.num_heads / a.qh), gy = (unsigned)a.split.nch;
     const bool pf = a.pf && 2 * (int64_t)gx * gy <= a.cus;
     const dim3 grid(gx, gy, pf ? 1u + (unsigned)kAttnPfPlanes : 1u);
-    const int v = attn_variant(a.head_dim, a.qh, a.max_seq, a.nch);
+    const int v = attn_variant(a);
     switch (a.head_dim) {
         case 64: return launch_attn_hd<64>(a, v, grid, st);
         case 128: return launch_attn_hd<128>(a, v, grid, st);

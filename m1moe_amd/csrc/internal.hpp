@@ -313,9 +313,9 @@ struct MvArgs {
 
 // Decode attention of one query position.  Workgroup (g, c): q heads
 // g*qh .. g*qh+qh-1 (one kv head) over positions c*n .. (c+1)*n - 1, n =
-// attn_chunk(positions, nch) of the launch's own positions (nch =
-// attention_chunks(max_seq, groups, cus) workgroups per group, at most
-// kAttnMaxChunks).
+// attn_chunk(positions, split.nch) of the launch's own positions, or all of up to
+// split.one (split = attention_split(max_seq, ...): split.nch workgroups per
+// group, at most kAttnMaxChunks).
 //   fused = 1: q, k_new, v_new are the raw projections of the current token;
 //     q and k get the per-head RMSNorm (q_norm/k_norm non-null) and RoPE at
 //     p = *pos, the new k/v row is stored at cache row p (flag 32 and no
@@ -323,6 +323,11 @@ struct MvArgs {
 //   fused = 0: q final, positions 0..seq_len-1 all from the caches.
 // The last workgroup of each group merges the chunks into out; counters
 // ([groups]) are back at 0 when the kernel ends.
+// (split: up to `one` positions are one workgroup's, more are shared evenly by
+// nch, at least kAttnChunk each; one > kAttnChunk goes with defer = 0)
+struct AttnSplit {
+    int32_t nch, one;
+};
 struct AttnArgs {
     int32_t fused;
     const float* q;              // [num_heads][head_dim]
@@ -341,7 +346,7 @@ struct AttnArgs {
     int32_t seq_len;             // fused = 0
     int32_t max_seq;             // cache rows (fused) / seq_len
     int32_t num_heads, num_kv_heads, hpkv, head_dim, qh;
-    int32_t nch;                 // workgroups per group (attention_chunks)
+    AttnSplit split;             // attention_split of max_seq
     float scale, rope_theta, eps;
     // fused only: for 2 .. kAttnDeferChunks active chunks and num_heads x chunks
     // <= kAttnDeferHeadChunks, write the partials and leave their merge to the
@@ -456,13 +461,11 @@ int matvec_rows_per_workgroup(int rows);
 int launch_matvec_bf16(const MvArgs& a, void* stream);
 // q heads per attention workgroup (0: unsupported hpkv).
 int attention_qh(int hpkv);
-// Attention workgroups per group for a cache of max_positions, groups
-// (num_heads / qh) and cus compute units: one per kAttnChunk positions while
-// they fit the CUs, then as many as fill the CUs once; at most kAttnMaxChunks.
-int attention_chunks(int max_positions, int groups, int cus);
-int attention_max_chunks(int max_positions);   // the most it gives, for any groups
-// Positions per workgroup of a launch over `positions` with nch workgroups per
-// group.
+// How the decode attention of groups (num_heads / qh) of qh heads shares up to
+// max_positions positions among workgroups on cus compute units.
+AttnSplit attention_split(int max_positions, int groups, int cus, int qh, int head_dim);
+int attention_max_chunks(int max_positions);   // the most workgroups per group it gives
+// Positions per workgroup of a launch over `positions` that nch workgroups share.
 M1MOE_HD inline int attn_chunk(int positions, int nch) {
     const int n = (positions + nch - 1) / nch;
     return n > kAttnChunk ? n : kAttnChunk;

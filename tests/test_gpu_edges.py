@@ -112,7 +112,11 @@ def test_router_tokens_per_wave(name, T):
     (32, 8, 128, 65), (32, 8, 128, 17), (24, 8, 64, 9), (300, 300, 64, 333), (2, 2, 256, 2),
     # eight heads per group: half a batch per wave, a whole one, the larger one
     (8, 1, 128, 1), (8, 1, 128, 32), (8, 1, 128, 33), (64, 8, 128, 2049), (64, 8, 128, 2560),
-    (8, 1, 256, 31), (8, 1, 256, 33), (8, 1, 256, 64), (16, 2, 256, 129)])
+    (8, 1, 256, 31), (8, 1, 256, 33), (8, 1, 256, 64), (16, 2, 256, 129),
+    # one workgroup per group up to 256, 320, 512 positions; more groups than CUs: one up to
+    # 256, chunks in the light forms, then of at least 256
+    (100, 100, 64, 512), (100, 100, 64, 513), (86, 86, 128, 320), (86, 86, 128, 321), (70, 70, 128, 257),
+    (128, 64, 128, 256), (260, 260, 64, 256), (260, 260, 64, 257), (260, 260, 64, 3073), (260, 260, 128, 1281)])
 def test_attention_decode_chunk_edges(ops_ctx, nh, nkv, hd, sl):
     """f32 sums of at most 8191 terms against the oracle's f64: 1e-6 (2e-7
     seen), for lengths around every batch and chunk rule; the last V row is
@@ -269,6 +273,34 @@ def test_decoder_steps_eight_heads_per_group(hd):
                 _, w_lg = p.orc.step(int(t))
                 assert rel_l2(g_lg, w_lg) < 1e-5
             at = stop + steps
+    finally:
+        p.close()
+
+
+@pytest.mark.parametrize("heads,kv,hd,steps", [(24, 24, 64, (2, 62, 126, 254, 256, 258)), (32, 16, 128, (126, 128)),
+                                               (32, 32, 128, (255, 256))])
+def test_decoder_steps_around_one_workgroup(heads, kv, hd, steps):
+    """Steps of a long cache around the positions up to which one workgroup takes
+    all of a group (256; 128 with 16 groups of two), with the early and the shared
+    forms on both sides."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    wl = synth.DecoderWorkload("one", synth.CONFIGS["tiny"], 1, 300, heads, kv, hd, 1e4, True, 8, 8)
+    p = Pair(wl, seed=66, max_seq=4000)
+    try:
+        _zero_experts(p)
+        toks = synth.prompt_tokens(wl, 10, 300)
+        at = 0
+        for stop in steps:
+            say(f"{heads}/{kv}/{hd}: step at {stop}")
+            if stop > at:
+                p.dec.prefill(toks[at:stop])
+            for t in toks[at:stop]:
+                p.orc.step(int(t))
+            _, g_lg = p.dec.forward(int(toks[stop]), return_logits=True)
+            _, w_lg = p.orc.step(int(toks[stop]))
+            assert rel_l2(g_lg, w_lg) < 1e-5
+            at = stop + 1
     finally:
         p.close()
 
