@@ -137,10 +137,9 @@ __global__ __launch_bounds__(256) void rope_kv_rows_kernel(PfDenseArgs a) {
     constexpr int kSlots = 256 / G, PASS = (kRopeHeads + kSlots - 1) / kSlots;
     const int t = blockIdx.x, slot = threadIdx.x / G, i = threadIdx.x % G;
     const int p = *a.pos + t, heads = a.num_heads + a.num_kv_heads;
-    if (p >= a.max_seq) {
-        if (threadIdx.x == 0 && blockIdx.y == 0) flag_error(a.err, 32u);
-        return;
-    }
+    const bool past = p >= a.max_seq;
+    if (past && threadIdx.x == 0 && blockIdx.y == 0) flag_error(a.err, 32u);
+    if (past && a.splits <= 1) return;
     // value at column c of the token's projections
     const size_t at = (size_t)t * a.ldqkv, step = (size_t)a.T * a.ldqkv;
     auto value = [&](int c) {
@@ -162,6 +161,10 @@ __global__ __launch_bounds__(256) void rope_kv_rows_kernel(PfDenseArgs a) {
         const bool is_q = head < a.num_heads;
         const int kvh = head - a.num_heads;
         const int c0 = is_q ? head * HD : a.qd + kvh * HD;
+        if (past) {   // (flagged) no row of the table or the caches; the query as it was projected
+            for (int d = i; is_q && d < HD; d += G) a.qkv[at + c0 + d] = value(c0 + d);
+            continue;
+        }
         const uint16_t* nw = is_q ? a.q_norm : a.k_norm;
         float x0[NP], x1[NP], v0[NP], v1[NP];
         float2 r[NP];

@@ -343,6 +343,36 @@ def test_prefill_attention_tile_edges(heads, kv, hd, Ts):
         p.close()
 
 
+def test_prefill_past_the_cache_reads_its_own_queries():
+    """Tokens past the cache's end are reported; their logits come from this
+    call's projections, not from what an earlier prompt left in the scratch
+    (hidden 512: the q/k/v GEMM leaves split partials, summed by the RoPE rows)."""
+    import m1moe_amd as m
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    moe = synth.Workload("wide", dict(hidden=512, num_experts=4, top_k=1, intermediate=64, group_size=64,
+                                      norm_topk_prob=False))
+    wl = synth.DecoderWorkload("past", moe, 1, 300, 8, 2, 64, 1e4, True, 8, 8)
+    p = Pair(wl, seed=67, max_seq=16)
+    try:
+        _zero_experts(p)
+        found = []
+        for seed in (1, 2):
+            p.dec.prefill(synth.prompt_tokens(wl, seed, 16))
+            p.dec.reset()
+            p.dec.prefill(synth.prompt_tokens(wl, 3, 4))
+            toks, lg, nx = p.ctx.to_device(synth.prompt_tokens(wl, 4, 16)), p.ctx.alloc(4 * 300), p.ctx.alloc(16)
+            say(f"16 tokens at position 4 of 16, after prompt {seed}")
+            p.dec.prefill_device(toks, 16, nx, lg)
+            with pytest.raises(m.M1MoEError):
+                p.ctx.sync()
+            found.append(lg.download(np.float32, 300).copy())
+            p.dec.reset()
+        assert np.all(np.isfinite(found[0])) and np.array_equal(*found)
+    finally:
+        p.close()
+
+
 def test_prefill_attention_keys_past_the_split():
     """A K value of 3.397e38 rounds to infinity in bf16 (its parts would add up
     to NaN): the wave's blocks are multiplied on f32 MFMA instead.  eps 0 and
