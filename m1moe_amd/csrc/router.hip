@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(RouterArgs a) {
     // for a prefill, an extra row of workgroups (the last) makes the f16 copy:
     // wave w < TT takes token t0 + w, beside the logits of the other rows
     if (a.xq && blockIdx.y == gridDim.y - 1) {
-        if (wave < TT) prep_token(a, t0 + wave, lane);
+        if (TT == 4 || wave < TT) prep_token(a, t0 + wave, lane);   // (four waves)
         return;
     }
     if (e0 >= a.E) return;
