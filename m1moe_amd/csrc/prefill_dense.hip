@@ -527,7 +527,9 @@ GemmPlan gemm_plan(const GemmArgs& g) {
     const long gm64 = (g.M + 63) / 64, gn128 = (g.N + 127) / 128, gn64 = (g.N + 63) / 64;
     const long big = (long)((g.M + 127) / 128) * ((g.N + 255) / 256);
     GemmPlan p{};
-    p.wide = !g.W1 || (g.n1 % 128 == 0 && g.n2 % 128 == 0);
+    // (instead of one column of tiles, two narrow ones: one layer of hidden 128 at 5 /
+    // 1000 tokens 55.2 -> 54.0, 83.2 -> 81.8 us a prompt)
+    p.wide = g.N > 128 && (!g.W1 || (g.n1 % 128 == 0 && g.n2 % 128 == 0));
     p.big = big > 208 && big <= 256 && (!g.W1 || (g.n1 % 256 == 0 && g.n2 % 256 == 0));
     const long tiles = p.wide ? gn128 * gm64 : gn64 * gm64, nkb = g.K / 64;
     long S = !p.big && g.part && tiles < 256 ? std::min(kGemmSplitWgs / tiles, nkb / 4) : 1;
