@@ -229,7 +229,7 @@ int32_t enqueue_router(m1moe_ctx_t ctx, int32_t layer, int32_t T, const void* x,
     r.counters = ctx->counters;
     r.xq = xq;
     r.xinv = xinv;
-    return launched(m1moe::launch_router_topk(r, ctx->stream), "router_topk");
+    return launched(m1moe::launch_router_topk(r, ctx->cus, ctx->stream), "router_topk");
 }
 
 // Sizes in bytes of the kPfBufs prefill scratch buffers for T tokens, in the

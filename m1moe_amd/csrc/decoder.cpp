@@ -100,7 +100,7 @@ struct m1moe_dec {
     float *pf_res = nullptr, *pf_res2 = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr;
     uint16_t* pf_parts = nullptr;  // GEMM inputs as three bf16 parts, [3][T][max(h, qd)]: the normed
                                    // rows, then the attention output
-    float* pf_part = nullptr;  // split-K partials of the prefill GEMMs (kGemmPartFloats)
+    float* pf_part = nullptr;  // split-K partials of the prefill GEMMs (gemm_part_floats)
     uint32_t* cnt = nullptr;   // [dec_cnt_words]: (unused) x 2, attention groups, the
                                // attention's launch number, then (dec_fin_offset) its
                                // finish counts and (dec_lm_offset) lm_head's
@@ -589,7 +589,7 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
             (rc = device_alloc((void**)&dec->pf_xn, t * h * 4, "prefill normed rows")) ||
             (rc = device_alloc((void**)&dec->pf_qkv, t * N * 4, "prefill q/k/v")) ||
             (rc = device_alloc((void**)&dec->pf_parts, t * std::max(h, qd) * 6, "prefill GEMM inputs")) ||
-            (rc = device_alloc((void**)&dec->pf_part, kGemmPartFloats * 4, "prefill split-K partials")))
+            (rc = device_alloc((void**)&dec->pf_part, (uint64_t)gemm_part_floats(ctx->cus) * 4, "prefill split-K partials")))
             return rc;
         dec->pf_cap = T;
     }
@@ -636,6 +636,7 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
         g.N = N;
         g.K = h;
         g.part = dec->pf_part;
+        g.cus = ctx->cus;
         // (split partials are summed by launch_pf_rope_kv)
         a.part = dec->pf_part;
         a.splits = gemm_splits(g);
@@ -671,6 +672,7 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
         o.N = h;
         o.K = qd;
         o.part = dec->pf_part;
+        o.cus = ctx->cus;
         o.norm_w = dec->post_norm + (size_t)l * h;
         o.norm_out = dec->pf_xn;
         o.norm_eps = eps;

@@ -229,7 +229,7 @@ constexpr uint64_t kStaticScratchBytes = 64ull << 20;
 int static_scratch_attach(int device, uint8_t** out);
 
 // launchers (defined next to their kernels); return a hipError_t as int
-int launch_router_topk(const RouterArgs& a, void* stream);
+int launch_router_topk(const RouterArgs& a, int cus, void* stream);
 int launch_moe_decode(const FusedArgs& a, void* stream);
 // The one-workgroup-per-CU decode kernel: the shapes it takes (hidden 2048,
 // K * I = 8192 or 16384, I = 1024 or 2048, K <= 8 dividing 8) and its
@@ -397,12 +397,13 @@ struct GemmArgs {
     float* C;
     int32_t ldc;
     int32_t M, N, K;
-    // split-K workspace ([S][M][N] f32 partials, to be summed in the order s =
-    // 0 .. S-1) or null; with it a GEMM whose tiles leave the CUs idle splits
+    // split-K workspace (gemm_part_floats; [S][M][N] f32 partials, to be summed in
+    // the order s = 0 .. S-1) or null; with it a GEMM whose tiles leave the CUs idle splits
     // its k range (gemm_splits).  With norm_w launch_gemm sums them into C,
     // without it they are left for the caller's next launch
     float* part;
     int32_t splits;              // set by launch_gemm
+    int32_t cus;                 // compute units
     // optional second and third weight segments: rows [n1, n2) are rows
     // 0 .. of W1, rows [n2, N) rows 0 .. of W2 (q, k and v in one launch);
     // null W1: every row from W.  n1 and n2 are multiples of 64.
@@ -417,7 +418,6 @@ struct GemmArgs {
     float norm_eps;
 };
 constexpr int kGemmMaxSplits = 8;
-constexpr int64_t kGemmPartFloats = 768LL * 64 * 64;  // the workspace launch_gemm may use
 
 // The T prompt tokens of a decoder prefill at positions *pos .. *pos + T - 1.
 struct PfDenseArgs {
@@ -449,6 +449,7 @@ int launch_rmsnorm_rows(const float* x, const uint16_t* w, float* out, uint16_t*
 int launch_gemm(const GemmArgs& g, void* stream);
 // The k splits launch_gemm makes of g (1: C is written by the GEMM itself).
 int gemm_splits(const GemmArgs& g);
+int64_t gemm_part_floats(int cus);
 int launch_pf_rope_kv(const PfDenseArgs& a, void* stream);
 int launch_pf_attention(const PfDenseArgs& a, void* stream);
 int launch_advance_pos(int32_t* pos, int32_t by, int32_t max_seq, void* stream);

@@ -477,8 +477,6 @@ __global__ __launch_bounds__(256) void splitk_sum_norm_kernel(GemmArgs g) {
     for (int i = threadIdx.x; i < g.N; i += 256) o[i] = c[i] * rms * bf16_to_f32(g.norm_w[i]);
 }
 
-constexpr long kGemmSplitWgs = 512;   // workgroups of a split grid
-
 }  // namespace
 
 int launch_pf_embed(const PfDenseArgs& a, void* stream) {
@@ -509,16 +507,23 @@ void launch_gemm_tile(const GemmArgs& g, hipStream_t st) {
 }
 }  // namespace
 
+int64_t gemm_part_floats(int cus) { return 3LL * cus * 64 * 64; }
+
 namespace {
 // Tiles of 64 x 128, two workgroups per CU: measured best or within a few
-// percent at every size but one, a grid of 128 x 256 tiles that is nearly one
-// full round of the CUs (2048 x 4096 x 4096: 256 of them 200 us, 1024 of 64 x
-// 128 215; 1100 x 6144 x 4096, 216: 175 against 207; but 192 of them at 1000 x
-// 6144 x 2048 84 against 82, 384 at 2048 x 6144 x 4096 342 against 307).  The
-// weight segments' borders must be tile borders.  Too few tiles: the k-blocks
-// are split over gridDim.y (at least 4 blocks of 64 per split, at most
-// kGemmSplitWgs workgroups in all) and the partials summed in a fixed order,
-// so results do not depend on timing.
+// percent at every size but one, a grid of 128 x 256 tiles that is more than
+// three quarters of one round of the CUs (of 256, M x N x K: 256 of them, 2048 x
+// 4096 x 4096, 200 us, 1024 of 64 x 128 215; 216, 1100 x 6144 x 4096, 175 against
+// 207; four layers of 1280 x 5120 x 4096, 200, a prompt 1823 against 1935 us; but 192
+// at 1000 x 6144 x 2048 84 against 82, 384 at 2048 x 6144 x 4096 342 against 307).
+// The weight segments' borders must be tile borders.  Fewer tiles than CUs: the
+// k-blocks are split over gridDim.y (at least 4 blocks of 64 per split: 6 of them
+// 279 -> 291 us a prompt of 17 tokens, hidden 1536, four layers; at most two
+// workgroups per CU and gemm_part_floats of partials in all) and the partials summed
+// in a fixed order, so results do not depend on timing.  The workspace's 12 MB is
+// what limits the splits from 384 workgroups of whole tiles on; with 16 MB, two per
+// CU, four layers of hidden 4096 would take 657 us in place of 677 at 128 tokens, 854
+// in place of 948 at 300, of hidden 2048 440 in place of 445 at 128.
 struct GemmPlan {
     bool big, wide;
     int splits;
@@ -530,10 +535,10 @@ GemmPlan gemm_plan(const GemmArgs& g) {
     // (instead of one column of tiles, two narrow ones: one layer of hidden 128 at 5 /
     // 1000 tokens 55.2 -> 54.0, 83.2 -> 81.8 us a prompt)
     p.wide = g.N > 128 && (!g.W1 || (g.n1 % 128 == 0 && g.n2 % 128 == 0));
-    p.big = big > 208 && big <= 256 && (!g.W1 || (g.n1 % 256 == 0 && g.n2 % 256 == 0));
+    p.big = 4 * big > 3 * g.cus && big <= g.cus && (!g.W1 || (g.n1 % 256 == 0 && g.n2 % 256 == 0));
     const long tiles = p.wide ? gn128 * gm64 : gn64 * gm64, nkb = g.K / 64;
-    long S = !p.big && g.part && tiles < 256 ? std::min(kGemmSplitWgs / tiles, nkb / 4) : 1;
-    S = std::min({S, (long)kGemmMaxSplits, (long)(kGemmPartFloats / ((int64_t)g.M * g.N))});
+    long S = !p.big && g.part && tiles < g.cus ? std::min(2 * g.cus / tiles, nkb / 4) : 1;
+    S = std::min({S, (long)kGemmMaxSplits, (long)(gemm_part_floats(g.cus) / ((int64_t)g.M * g.N))});
     p.splits = (int)std::max(S, 1l);
     return p;
 }
@@ -545,7 +550,7 @@ int launch_gemm(const GemmArgs& g0, void* stream) {
     GemmArgs g = g0;
     if (g.K % 64 || g.K <= 0 || g.M <= 0 || g.N <= 0 || g.N % 4 || g.ldc % 4 || (uintptr_t)g.C % 16 ||
         (uintptr_t)g.R % 16 || g.xplane < (int64_t)g.M * g.K || 6 * g.xplane >= (1ll << 32) ||
-        2ll * 128 * g.K >= (1ll << 32))
+        2ll * 128 * g.K >= (1ll << 32) || g.cus <= 0)
         return (int)hipErrorInvalidValue;
     if (g.W1 && (!g.W2 || g.n1 < 0 || g.n1 > g.n2 || g.n2 > g.N || g.n1 % 64 || g.n2 % 64))
         return (int)hipErrorInvalidValue;

@@ -256,8 +256,6 @@ __global__ __launch_bounds__(256) void router_rank_kernel(RouterArgs a) {
     }
 }
 
-constexpr long kFewWorkgroups = 256;   // one per CU
-
 template <int TT>
 void launch_logits(const RouterArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(router_logits_kernel<TT>,
@@ -268,7 +266,7 @@ void launch_logits(const RouterArgs& a, hipStream_t st) {
 
 }  // namespace
 
-int launch_router_topk(const RouterArgs& a, void* stream) {
+int launch_router_topk(const RouterArgs& a, int cus, void* stream) {
     if (a.E > kMaxE || a.K > kMaxK || a.h % 64) return (int)hipErrorInvalidValue;
     hipStream_t st = static_cast<hipStream_t>(stream);
     // The fewest tokens per wave whose grid fits the CUs once: a short prompt's
@@ -277,9 +275,9 @@ int launch_router_topk(const RouterArgs& a, void* stream) {
     // 6.5), a long one's the loads and conversions that more tokens share (T =
     // 512 11.5 us at four, 13.9, 16.6; T = 1000 x 8 x 4096 15.7, 19.2, 17.6).
     const long groups = (a.E + kTE - 1) / kTE;
-    if (a.T * groups <= kFewWorkgroups)
+    if (a.T * groups <= cus)
         launch_logits<1>(a, st);
-    else if ((a.T + 1) / 2 * groups <= kFewWorkgroups)
+    else if ((a.T + 1) / 2 * groups <= cus)
         launch_logits<2>(a, st);
     else
         launch_logits<4>(a, st);
