@@ -343,6 +343,85 @@ def test_prefill_attention_tile_edges(heads, kv, hd, Ts):
         p.close()
 
 
+@pytest.mark.parametrize("heads,kv,qk_norm,Ts", [(2, 1, True, (17, 33)), (4, 4, False, (1, 16, 31)),
+                                                 (3, 1, True, (50,))])
+def test_prefill_head_dim_256(heads, kv, qk_norm, Ts):
+    """RoPE rows with two pairs per lane and the SIMD attention's outputs in pairs,
+    16-query tiles one short of, at and past their edge, behind an earlier
+    context; two layers, so that every query's output reaches the last logits."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    wl = synth.DecoderWorkload("hd256", synth.CONFIGS["tiny_renorm"], 2, 300, heads, kv, 256, 1e4, qk_norm, 8, 8)
+    p = Pair(wl, seed=68, max_seq=sum(Ts))
+    try:
+        _zero_experts(p)
+        _prefill_matches(p, synth.prompt_tokens(wl, 6, sum(Ts)), Ts)
+    finally:
+        p.close()
+
+
+@pytest.mark.parametrize("hidden", [4096, 4160, 8192])
+def test_prefill_row_norms_of_wide_rows(hidden):
+    """Both sides of the row norms' register forms (4096, 8192 values a row)."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    moe = synth.Workload("wide", dict(hidden=hidden, num_experts=2, top_k=1, intermediate=64, group_size=64,
+                                      norm_topk_prob=False))
+    wl = synth.DecoderWorkload("wide_rows", moe, 1, 300, 2, 1, 64, 1e4, True, 8, 8)
+    p = Pair(wl, seed=69, max_seq=12)
+    try:
+        _zero_experts(p)
+        _prefill_matches(p, synth.prompt_tokens(wl, 7, 12), (5, 7))
+    finally:
+        p.close()
+
+
+def test_prefill_large_gemm_tile_over_three_segments():
+    """1100 x 6144 x 512: nine rows of 24 tiles of 128 x 256 over q, k and v, the
+    last one ragged; K and V of every token reach the last logits."""
+    from test_gpu_decoder import Pair, _zero_experts
+    from m1moe_amd import synth
+    moe = synth.Workload("qkv", dict(hidden=512, num_experts=2, top_k=1, intermediate=64, group_size=64,
+                                     norm_topk_prob=False))
+    wl = synth.DecoderWorkload("segments", moe, 1, 300, 16, 16, 128, 1e4, True, 8, 8)
+    p = Pair(wl, seed=70, max_seq=1100)
+    try:
+        _zero_experts(p)
+        _prefill_matches(p, synth.prompt_tokens(wl, 8, 1100), (1100,))
+    finally:
+        p.close()
+
+
+def test_prefill_large_gemm_tile_ragged_with_residual():
+    """o_proj of 1700 x 4096 x 4096 (14 x 16 tiles of 128 x 256, the last row
+    ragged) with the residual and the row norm, against the same prompt in
+    pieces of 400 (64 x 128 tiles): f32 sums in another order, 1e-5.  Two layers, so
+    that every row reaches the last logits through the second layer's K and V."""
+    from m1moe_amd import synth
+    from m1moe_amd.decoder import Decoder
+    wl = synth.DECODERS["cfg4"]
+    shape = synth.Workload("wide", dict(hidden=4096, num_experts=2, top_k=1, intermediate=64, group_size=64,
+                                        norm_topk_prob=False)).shape(2)
+    ctx = m.HIPContext(shape)
+    try:
+        for l in range(2):
+            ctx.upload_layer_experts(l, np.zeros_like(synth.layer_image(shape, 71, l)))
+            ctx.upload_router(l, synth.router(shape, 71, l))
+        dec = Decoder(ctx, wl.dec_shape(1700))
+        dec.upload_all(lambda which, l: synth.dense_weight(wl, 71, which, l))
+        toks = synth.prompt_tokens(wl, 11, 1700)
+        say("1700 tokens at once")
+        _, whole = dec.prefill(toks, return_logits=True)
+        dec.reset()
+        for at in range(0, 1700, 400):
+            say(f"tokens from {at}")
+            _, pieces = dec.prefill(toks[at:at + 400], return_logits=True)
+        assert np.all(np.isfinite(whole)) and rel_l2(whole, pieces) < 1e-5
+        dec.close()
+    finally:
+        ctx.close()
+
+
 def test_prefill_past_the_cache_reads_its_own_queries():
     """Tokens past the cache's end are reported; their logits come from this
     call's projections, not from what an earlier prompt left in the scratch
