@@ -618,7 +618,6 @@ int32_t dec_prefill_piece(m1moe_dec_t dec, const int32_t* d_tokens, int32_t T,
     a.head_dim = hd;
     a.max_seq = dec->sh.max_seq;
     a.scale = 1.0f / sqrtf((float)hd);
-    a.rope_theta = dec->sh.rope_theta;
     a.eps = eps;
     // q, k and v of layer l: one launch over the three weight segments
     auto qkv_gemm = [&](int l) -> int32_t {

@@ -761,24 +761,6 @@ __device__ void attn_merge_share(const AttnArgs& a, int g, int c, int nch, int n
     if (mine && r == 0) a.out[(size_t)(g * QH + i) * HD + d] = acc / s_l[i];
 }
 
-
-// Workgroup (g, c): q heads g*QH .. g*QH+QH-1 (one kv head), positions
-// c*chunk .. (c+1)*chunk - 1.  Lanes take 8 dims of one position each (LP =
-// HD/8 lanes per position, 64/LP positions per wave and load), so every K or V
-// row is one coalesced read shared by the QH heads.  Each wave walks
-// batches of SB loads (V 1: batches wave, wave + 4, ... of the chunk, two in
-// flight; V 0 and 2: its quarter of the chunk as one batch of at most 4 or 5
-// loads, no second register set), and each of its 64/LP position groups keeps
-// a running softmax of its own (the softmax of attnSoftmax, Shaders.metal:245-289, in pieces), merged
-// across the wave's lanes and the waves only at the end of the chunk: no
-// barrier and no LDS between the first row and the last.  Bound by HBM at long
-// contexts (2 x kv_heads x head_dim x 4 bytes per position), by the chain
-// launch - rows - merge at short ones.  Against 64-position sub-chunks that all
-// four waves scored, normalised and summed between three barriers: 16 heads of
-// 128 at 200 / 2112 / 8192 positions 7.0 / 13.6 / 33.1 -> 6.7 / 12.2 / 29.7 us,
-// 32 q / 8 kv heads at 2112 / 5003 / 8192 12.0 / 30.6 / 24.7 -> 11.0 / 16.9 /
-// 20.5 us (5003 with its old 320 workgroups of 128 positions on 256 CUs; 41 MB
-// of rows in 16.9 us, 2.4 TB/s launch and merge included).
 // The planes z >= 1 of an attention grid: workgroup p of the P in them
 // (linear dispatch number A + p after the A attention workgroups, so XCD
 // p mod 8 when A and P are multiples of 8)
@@ -808,8 +790,8 @@ __device__ void attn_prefetch(const AttnArgs& a) {
     asm volatile("" ::"v"(acc));
 }
 
-// Loads per batch.  V 0: a quarter of 64 positions; V 2: of 96 (head_dim 64) or
-// 80 (128); V 1: what two register sets leave room for.
+// Loads per batch.  V 0: a quarter of 64 positions (2, 4 or 8 loads); V 2: of 96 (head_dim
+// 64, 3 loads) or 80 (128, 5); V 1: what two register sets leave room for.
 template <int HD, int QH, int V>
 __host__ __device__ constexpr int attn_sb() {
     return V == 0 ? HD / 32 : V == 2 ? HD / 32 + 1 : QH == 8 ? 2 : 4;
@@ -822,6 +804,23 @@ constexpr int attn_wgs() {
     return QH == 8 && HD == 256 && V == 0 ? 1 : 2;
 }
 
+// Workgroup (g, c): q heads g*QH .. g*QH+QH-1 (one kv head), positions
+// c*chunk .. (c+1)*chunk - 1.  Lanes take 8 dims of one position each (LP =
+// HD/8 lanes per position, 64/LP positions per wave and load), so every K or V
+// row is one coalesced read shared by the QH heads.  Each wave walks
+// batches of SB loads (V 1: batches wave, wave + 4, ... of the chunk, two in
+// flight; V 0 and 2: its quarter of the chunk as one batch, attn_sb loads, no
+// second register set), and each of its 64/LP position groups keeps
+// a running softmax of its own (the softmax of attnSoftmax, Shaders.metal:245-289, in pieces), merged
+// across the wave's lanes and the waves only at the end of the chunk: no
+// barrier and no LDS between the first row and the last.  Bound by HBM at long
+// contexts (2 x kv_heads x head_dim x 4 bytes per position), by the chain
+// launch - rows - merge at short ones.  Against 64-position sub-chunks that all
+// four waves scored, normalised and summed between three barriers: 16 heads of
+// 128 at 200 / 2112 / 8192 positions 7.0 / 13.6 / 33.1 -> 6.7 / 12.2 / 29.7 us,
+// 32 q / 8 kv heads at 2112 / 5003 / 8192 12.0 / 30.6 / 24.7 -> 11.0 / 16.9 /
+// 20.5 us (5003 with its old 320 workgroups of 128 positions on 256 CUs; 41 MB
+// of rows in 16.9 us, 2.4 TB/s launch and merge included).
 template <int HD, int QH, int V>
 __global__ __launch_bounds__(256, (attn_wgs<HD, QH, V>())) void attn_kernel(AttnArgs a) {
     if (blockIdx.z) {

@@ -438,7 +438,7 @@ struct PfDenseArgs {
     uint32_t* err;
     int32_t T, vocab, h, ldqkv, qd, kvd;
     int32_t num_heads, num_kv_heads, hpkv, head_dim, max_seq;
-    float scale, rope_theta, eps;
+    float scale, eps;
 };
 
 int launch_pf_embed(const PfDenseArgs& a, void* stream);

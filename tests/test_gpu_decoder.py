@@ -84,17 +84,16 @@ def test_matvec_bf16(ops_ctx, rows, cols, with_res):
                                            (16, 16, 128, 4096), (32, 8, 128, 2112),
                                            (32, 4, 128, 2112), (16, 2, 64, 4096),
                                            (8, 2, 128, 5000), (4, 4, 64, 8300),
-                                           # one wide sub-chunk per workgroup (65..80
+                                           # one larger batch per wave (chunks of 65..80
                                            # positions: the grid fits the CUs)
                                            (32, 8, 64, 2100), (32, 8, 256, 2100),
                                            (64, 64, 128, 300)])
 def test_attention_decode(ops_ctx, nh, nkv, hd, sl):
     """The attention building block against the oracle: one chunk, 64-position
-    chunks up to 64 per kv head, chunks of several 64-position sub-chunks
-    (two K/V register sets), chunks of one wide sub-chunk (65..80
-    positions, when 64-position chunks would put more workgroups than CUs:
-    the Mixtral grouping at 2100-2112 positions, 64 single-head groups at
-    300), head_dim 64 / 128 / 256."""
+    chunks up to 64 per kv head, longer ones walked in batches of loads with
+    two K/V register sets, chunks that are one larger batch per wave (65..80
+    positions: the Mixtral grouping at 2100-2112 positions, 64 single-head
+    groups at 300), head_dim 64 / 128 / 256."""
     ctx, ops = ops_ctx
     kvd = nkv * hd
     q = RNG.normal(0, 1, nh * hd).astype(np.float32)
@@ -395,11 +394,11 @@ def test_prefill_dense_path_is_tight(Ts):
 def test_prefill_split_k_gemms_are_tight():
     """OLMoE widths (h = q = kv = 2048), one layer, MoE block zeroed.  A
     100-token prefill: q, k and v as one launch over three weight segments
-    (192 tiles of 64 x 64, 4 shares of 8 k-blocks), o_proj 64 tiles in 8
-    shares of 4 k-blocks, summed with the residual and normalised in one
-    kernel; a second 200-token prefill: q/k/v 384 tiles in 2 shares, o_proj
-    128 tiles in 6 shares of 5-6 k-blocks.  Partials summed in a fixed order;
-    last logits against the oracle's token-by-token run to relative L2 1e-5."""
+    (96 tiles of 64 x 128, 5 shares of 6-7 k-blocks, summed by the RoPE rows),
+    o_proj 32 tiles in 8 shares of 4 k-blocks, summed with the residual and
+    normalised in one kernel; a second 200-token prefill: q/k/v 192 tiles in 2
+    shares, o_proj 64 tiles in 7 shares of 4-5 k-blocks (what the workspace
+    holds).  Partials summed in a fixed order; last logits against the oracle's token-by-token run to relative L2 1e-5."""
     p = Pair(synth.DECODERS["cfg1"], seed=53, max_seq=310, num_layers=1, nthreads=8)
     try:
         _zero_experts(p)
@@ -441,7 +440,7 @@ def test_prefill_longer_than_one_piece():
 @pytest.mark.parametrize("Ts", [(150,), (40, 90)])
 def test_prefill_dense_path_head_dim_128_gqa(Ts):
     """The MFMA prefill attention at head_dim 128 with 4 q heads per kv head
-    (the Mixtral grouping), T crossing several 64-query and 32-key blocks,
+    (the Mixtral grouping), T crossing several 32-query and 32-key blocks,
     a second prefill over a past context: last logits against the oracle's
     token-by-token run to relative L2 1e-5 (MoE block zeroed)."""
     wl = synth.DecoderWorkload("hd128_gqa", synth.CONFIGS["tiny_renorm"], 1, 300, 8, 2, 128,
