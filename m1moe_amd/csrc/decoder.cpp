@@ -32,7 +32,8 @@ uint64_t dec_fin_offset(int num_heads) { return 32 * ((3 + (uint64_t)num_heads +
 uint64_t dec_lm_offset(int num_heads) { return dec_fin_offset(num_heads) + kCountWords; }
 uint64_t dec_cnt_words(int num_heads) { return dec_lm_offset(num_heads) + kCountWords; }
 
-int32_t ensure_attn_scratch(m1moe_ctx_t ctx, uint64_t floats) {
+// At least `floats` of attention scratch; a new buffer has `reserve` if that is more.
+int32_t ensure_attn_scratch(m1moe_ctx_t ctx, uint64_t floats, uint64_t reserve) {
     ctx->capture_uses_scratch = true;
     if (!ctx->attn_cnt || floats > ctx->attn_part_floats)
         if (int32_t rc = refuse_growth_in_capture(ctx->stream, "the attention scratch")) return rc;
@@ -42,6 +43,7 @@ int32_t ensure_attn_scratch(m1moe_ctx_t ctx, uint64_t floats) {
         HIP_TRY(hipMemsetAsync(ctx->attn_cnt, 0, kAttnCntWords * 4, ctx->stream));
     }
     if (floats <= ctx->attn_part_floats) return M1MOE_OK;
+    floats = std::max(floats, reserve);
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     if (ctx->attn_part) ++ctx->scratch_gen;  // earlier graphs hold the old buffer
     if (ctx->attn_part) HIP_TRY(hipFree(ctx->attn_part));
@@ -214,11 +216,14 @@ int32_t m1moe_attention_decode(m1moe_ctx_t ctx, const float* d_q, const float* d
     a.qh = attention_qh(num_heads / num_kv_heads);
     a.cus = ctx->cus;
     a.split = attention_split(seq_len, num_heads / a.qh, a.cus, a.qh, head_dim);
-    // (for the most chunks any head count has over these positions: the scratch
-    // is the context's, and a shape that a graph is captured with may follow
-    // another one of as many heads and positions)
-    const int32_t most = attention_max_chunks(seq_len);
-    if ((rc = ensure_attn_scratch(ctx, attention_partial_floats(num_heads, head_dim, most)))) return rc;
+    // (a new buffer also holds the most chunks any grouping of the heads has over
+    // these positions: the scratch is the context's, and a shape that a graph is
+    // captured with may follow another one of as many heads and positions; up to
+    // 1 MiB: from 2 MiB on the first call takes 20 to 100 us longer)
+    const uint64_t most = (uint64_t)attention_partial_floats(num_heads, head_dim, attention_max_chunks(seq_len));
+    if ((rc = ensure_attn_scratch(ctx, (uint64_t)attention_partial_floats(num_heads, head_dim, a.split.nch),
+                                  std::min<uint64_t>(most, (1u << 20) / 4))))
+        return rc;
     a.fused = 0;
     a.q = d_q;
     a.kcache = const_cast<float*>(d_kcache);  // read only when fused = 0

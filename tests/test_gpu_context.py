@@ -120,7 +120,7 @@ def test_graph_refused_after_scratch_growth():
 
 def test_attention_capture_after_another_head_count():
     """The attention scratch that one call made covers every other grouping of
-    as many heads over as many positions: the first call of 32 q / 4 kv heads is
+    as many heads over as many positions (as far as 1 MiB holds it): the first call of 32 q / 4 kv heads is
     captured (a graph may not grow scratch), and a graph of the 32-head form
     stays valid after it."""
     from m1moe_amd.decoder import DenseOps
