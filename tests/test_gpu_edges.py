@@ -104,8 +104,9 @@ def test_router_tokens_per_wave(name, T):
 
 @pytest.mark.parametrize("nh,nkv,hd,sl", [
     # 64 groups on 256 CUs: four workgroups each, chunks of 64 (one batch per wave),
-    # 65 .. 96 or 80 (one larger batch) and above (two batches in flight)
-    (64, 64, 64, 256), (64, 64, 64, 257), (64, 64, 64, 384), (64, 64, 64, 385),
+    # 65 .. 96 or 80 (one larger batch) and above (two batches in flight; at head_dim 64
+    # 385 .. 512 positions are one workgroup's)
+    (64, 64, 64, 256), (64, 64, 64, 257), (64, 64, 64, 384), (64, 64, 64, 385), (64, 64, 64, 513),
     (64, 64, 128, 255), (64, 64, 128, 320), (64, 64, 128, 321), (64, 64, 256, 256),
     (64, 64, 256, 259), (64, 8, 64, 2049), (64, 8, 128, 130), (64, 8, 128, 8191),
     # one position past a chunk, past a wave's batch; more groups than CUs
